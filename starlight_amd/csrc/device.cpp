@@ -761,6 +761,138 @@ size_t try_fuse(Device* d, size_t i, hipError_t* err) {
     return 0;
 }
 
+// The same units on dense f32 weights, for at most 32 rows (decode):
+// [RmsNorm +] up to three MatMulNT reading the same rows, or one MatMulNT +
+// the residual Add, or [RmsNorm +] SwiGlu [+ the residual Add], as one dense
+// GEMV launch each (two for SwiGlu). Blocks of a launch write outputs while
+// others still read the weights, so no output may overlap a weight of the
+// launch either. Returns the commands covered (0: nothing launched).
+size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
+    const size_t n = d->log.size();
+    const Logged* norm = nullptr;
+    size_t j = i;
+    if (d->log[i].plan.code == SL_OP_RMS_NORM) {
+        norm = &d->log[i];
+        j = i + 1;
+        if (j >= n || overlaps(norm->out, norm->in[0]) || overlaps(norm->out, norm->in[1])) return 0;
+    }
+    const Logged& c1 = d->log[j];
+    if (norm && !same_ref(c1.in[0], norm->out)) return 0;
+    const sl_buffer_ref a_ref = norm ? norm->in[0] : c1.in[0];
+    // everything a launch of the unit reads or its prologue writes
+    sl_buffer_ref touched[3 + kFusedMaxSegs] = {a_ref, norm ? norm->in[1] : a_ref, norm ? norm->out : a_ref};
+    size_t n_touched = 3;
+    const auto clashes = [&](const sl_buffer_ref& r) {
+        for (size_t t = 0; t < n_touched; ++t)
+            if (overlaps(r, touched[t])) return true;
+        return false;
+    };
+    GemvDense f{};
+    f.a = fptr(d, a_ref);
+    f.epilogue = kFusedPlain;
+    if (norm) {
+        f.gamma = fptr(d, norm->in[1]);
+        f.normed = fptr(d, norm->out);
+        f.eps = norm->plan.eps;
+    }
+    // the norm inside the GEMV's prologue, or ahead of it on its own
+    const auto run = [&]() -> hipError_t {
+        if (!norm || gemv_dense_norm_takes(f)) return launch_gemv_dense(f, d->stream);
+        const hipError_t e = launch_rms_norm(f.a, f.gamma, f.normed, f.m, f.k, f.eps, d->stream);
+        if (e != hipSuccess) return e;
+        f.a = f.normed;
+        f.gamma = nullptr;
+        return launch_gemv_dense(f, d->stream);
+    };
+
+    if (c1.plan.code == SL_OP_MATMUL_NT && !c1.plan.quant[1].present) {
+        const uint64_t rows = c1.plan.batch * c1.plan.m, k = c1.plan.k;
+        if (rows == 0 || (norm && (norm->plan.rows != rows || norm->plan.hidden != k))) return 0;
+        f.m = rows;
+        f.k = k;
+        sl_buffer_ref outs[kFusedMaxSegs];
+        uint32_t cnt = 0;
+        for (size_t t = j; t < n && cnt < kFusedMaxSegs; ++t) {
+            const Logged& c = d->log[t];
+            if (c.plan.code != SL_OP_MATMUL_NT || c.plan.quant[1].present || !same_ref(c.in[0], c1.in[0]) ||
+                c.plan.batch * c.plan.m != rows || c.plan.k != k || c.plan.batch_b != 1 ||
+                c.plan.batch_a != c.plan.batch)
+                break;
+            bool clash = clashes(c.out);
+            for (uint32_t x = 0; x < cnt; ++x) clash = clash || overlaps(c.out, outs[x]) || overlaps(c.in[1], outs[x]);
+            if (clash || (norm && overlaps(c.in[1], norm->out))) break;
+            touched[n_touched++] = c.in[1];
+            f.w[cnt] = fptr(d, c.in[1]);
+            f.n[cnt] = c.plan.n;
+            f.out[cnt] = fptr(d, c.out);
+            outs[cnt] = c.out;
+            ++cnt;
+        }
+        if (cnt == 0) return 0;
+        f.nseg = cnt;
+        size_t used = (j - i) + cnt;
+        if (cnt == 1 && j + 1 < n) {
+            const Logged& add = d->log[j + 1];
+            const int other = residual_port(add, outs[0], rows * f.n[0], touched, n_touched, norm ? &norm->out : nullptr);
+            if (other >= 0) {
+                f.epilogue = kFusedResidual;
+                f.resid[0] = fptr(d, add.in[other]);
+                f.out2[0] = fptr(d, add.out);
+                ++used;
+            }
+        }
+        if (used == 1 || !gemv_dense_takes(f)) return 0;
+        *err = run();
+        d->stats.fused_commands += used;
+        return used;
+    }
+
+    if (c1.plan.code == SL_OP_SWIGLU && !c1.plan.quant[1].present && !c1.plan.quant[2].present &&
+        !c1.plan.quant[3].present) {
+        const uint64_t rows = c1.plan.rows, hidden = c1.plan.hidden, inter = c1.plan.inter;
+        if (rows == 0 || rows * inter > d->workspace_floats ||
+            (norm && (norm->plan.rows != rows || norm->plan.hidden != hidden ||
+                      overlaps(norm->out, c1.in[1]) || overlaps(norm->out, c1.in[2]))))
+            return 0;
+        float* h = d->workspace;
+        f.m = rows;
+        f.k = hidden;
+        f.nseg = 2;
+        f.epilogue = kFusedPair;
+        for (int t = 0; t < 2; ++t) {
+            f.w[t] = fptr(d, c1.in[1 + t]);
+            f.n[t] = inter;
+        }
+        f.out[0] = h;
+        GemvDense g{};
+        g.a = h;
+        g.w[0] = fptr(d, c1.in[3]);
+        g.n[0] = hidden;
+        g.out[0] = fptr(d, c1.out);
+        g.nseg = 1;
+        g.m = rows;
+        g.k = inter;
+        g.epilogue = kFusedPlain;
+        if (!gemv_dense_takes(f) || !gemv_dense_takes(g)) return 0;
+        size_t used = (j - i) + 1;
+        if (j + 1 < n) {
+            const Logged& add = d->log[j + 1];
+            const int other = residual_port(add, c1.out, rows * hidden, &c1.in[3], 1);
+            if (other >= 0) {
+                g.epilogue = kFusedResidual;
+                g.resid[0] = fptr(d, add.in[other]);
+                g.out2[0] = fptr(d, add.out);
+                ++used;
+            }
+        }
+        *err = run();
+        if (*err == hipSuccess) *err = launch_gemv_dense(g, d->stream);
+        d->stats.fused_commands += used;
+        return used;
+    }
+    return 0;
+}
+
 const uint32_t* dyn_of(const Device* d, const Logged& c) {
     return c.dyn_slot >= 0 ? d->dyn + c.dyn_slot : nullptr;
 }
@@ -1037,6 +1169,7 @@ hipError_t run_log(Device* d) {
         if (d->options & SL_HIP_OPT_FUSION) {
             used = try_fuse_attention(d, i, &e);
             if (used == 0 && e == hipSuccess) used = try_fuse(d, i, &e);
+            if (used == 0 && e == hipSuccess) used = try_fuse_dense(d, i, &e);
             if (used == 0 && e == hipSuccess) used = try_fuse_silu_mul(d, i, &e);
         }
         if (e != hipSuccess) return e;

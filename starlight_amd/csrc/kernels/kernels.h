@@ -31,6 +31,7 @@ struct Workspace {
 // them all and returns the first error.
 hipError_t load_code_attention();
 hipError_t load_code_elementwise();
+hipError_t load_code_gemv_dense();
 hipError_t load_code_layout();
 hipError_t load_code_matmul();
 hipError_t load_code_norm_softmax();
@@ -43,7 +44,7 @@ inline hipError_t preload_code() {
     hipError_t (*const loads[])() = {load_code_attention, load_code_elementwise, load_code_layout,
                                      load_code_matmul,    load_code_norm_softmax, load_code_qgemm_mfma,
                                      load_code_qgemv_fused, load_code_qgemv_mfma, load_code_qmatmul,
-                                     load_code_rope};
+                                     load_code_rope,      load_code_gemv_dense};
     hipError_t first = hipSuccess;
     for (auto load : loads) {
         const hipError_t e = load();
@@ -279,6 +280,30 @@ struct QgemvFused {
     uint64_t partial_floats = 0;
 };
 hipError_t launch_qgemv_fused(const QgemvFused& f, hipStream_t s);
+
+// MatMulNT on dense f32 weights for at most 32 activation rows, with the same
+// fusions (gemv_dense.hip): up to three weights [n, k] reading the same rows.
+// Needs k % 4 == 0 and 16-byte aligned a and weights; the norm prologue also
+// m <= 4, m * k <= 16384, k % 256 == 0 and aligned gamma and normed. Else
+// hipErrorNotSupported, nothing launched. kFusedPair takes two weights of
+// equal n. No output may overlap anything the launch reads.
+struct GemvDense {
+    const float* a;       // [m, k]
+    const float* gamma;   // RMSNorm weight [k] applied to a first, or null
+    float* normed;        // where the normalised a is written (gamma set), or null
+    float eps;
+    const float* w[kFusedMaxSegs];
+    uint64_t n[kFusedMaxSegs];
+    float* out[kFusedMaxSegs];
+    const float* resid[kFusedMaxSegs];
+    float* out2[kFusedMaxSegs];
+    uint32_t nseg;
+    uint64_t m, k;
+    uint32_t epilogue;
+};
+bool gemv_dense_takes(const GemvDense& f);
+bool gemv_dense_norm_takes(const GemvDense& f);
+hipError_t launch_gemv_dense(const GemvDense& f, hipStream_t s);
 
 // Weights are dense f32 (pointer) or quantized (QuantWeight with tiles != null).
 struct WeightRef {

@@ -193,6 +193,25 @@ __global__ __launch_bounds__(256) void sgemm_tiled(const float* __restrict__ a, 
 hipError_t launch_matmul(const float* a, const float* b, float* out, uint64_t batch, uint64_t batch_a,
                          uint64_t batch_b, uint64_t m, uint64_t k, uint64_t n, bool nt, hipStream_t s) {
     if (batch == 0 || m == 0 || n == 0) return hipSuccess;
+    if (nt && batch_b == 1 && batch_a == batch && batch > 1) {
+        // one B for every batch: the batches are more rows of A
+        m *= batch;
+        batch = batch_a = 1;
+    }
+    if (nt && batch == 1) {
+        // few rows: B streamed once (gemv_dense.hip)
+        GemvDense f{};
+        f.a = a;
+        f.w[0] = b;
+        f.n[0] = n;
+        f.out[0] = out;
+        f.nseg = 1;
+        f.m = m;
+        f.k = k;
+        f.epilogue = kFusedPlain;
+        const hipError_t e = launch_gemv_dense(f, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     const uint64_t a_stride = batch_a == 1 && batch > 1 ? 0 : m * k;
     const uint64_t b_stride = batch_b == 1 && batch > 1 ? 0 : n * k;
     // matrix cores: 16-byte rows (k % 4 == 0, and n % 4 == 0 for NN rows of
