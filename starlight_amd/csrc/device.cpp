@@ -61,6 +61,7 @@ struct Buffer {
     uint32_t scales = 0;
     uint8_t* tiles = nullptr;  // private codes, then (Mfma) tile-ordered scales
     float* tile_scales = nullptr;
+    uint8_t* fp6 = nullptr;  // 6-bit copy (its own allocation), where the weight has one
     QuantLayout layout = QuantLayout::RowMajor;
 };
 
@@ -209,6 +210,8 @@ sl_status copy_in(Device* d, uint32_t id, const void* data, size_t len, uint32_t
         // A re-uploaded quantized payload refreshes the private tile copy.
         e = launch_quant_repack(static_cast<const uint8_t*>(b.ptr), b.tiles, b.desc.qformat, b.desc.qn, b.desc.qk,
                                 b.layout, d->stream);
+        if (e == hipSuccess && b.fp6)
+            e = launch_fp6_repack(static_cast<const uint8_t*>(b.ptr), b.fp6, b.desc.qn, b.desc.qk, d->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(d->stream);
         if (e != hipSuccess) return d->hip_fail(e);
     }
@@ -280,6 +283,7 @@ WeightRef weight_ref(Device* d, const sl_buffer_ref& r, const QuantOperand& q) {
     w.quant.layout = b.layout;
     w.quant.scales = static_cast<const float*>(d->buffers[b.scales].ptr);
     w.quant.tile_scales = b.tile_scales;
+    w.quant.fp6 = b.fp6;
     w.quant.format = q.format;
     w.quant.group = q.group;
     w.quant.n = q.n;
@@ -1406,6 +1410,7 @@ void sl_hip_device_destroy(sl_hip_device* d) {
     for (auto& b : d->buffers) {
         if (b.base) (void)hipFree(b.base);
         if (b.tiles) (void)hipFree(b.tiles);
+        if (b.fp6) (void)hipFree(b.fp6);
     }
     if (d->workspace) (void)hipFree(d->workspace);
     if (d->rope_tab) (void)hipFree(d->rope_tab);
@@ -1672,8 +1677,10 @@ sl_status sl_hip_bind_quantized(sl_hip_device* d, uint32_t payload, uint32_t sca
     if (pb.tiles) {
         (void)hipStreamSynchronize(d->stream);
         (void)hipFree(pb.tiles);
+        if (pb.fp6) (void)hipFree(pb.fp6);
         pb.tiles = nullptr;
         pb.tile_scales = nullptr;
+        pb.fp6 = nullptr;
     }
     if (bytes != 0) {
         if (hipMalloc(reinterpret_cast<void**>(&pb.tiles), bytes) != hipSuccess) {
@@ -1682,6 +1689,12 @@ sl_status sl_hip_bind_quantized(sl_hip_device* d, uint32_t payload, uint32_t sca
             return d->fail(Error::out_of_memory(bytes / 4));
         }
         if (scale_floats) pb.tile_scales = reinterpret_cast<float*>(pb.tiles + scale_offset);
+    }
+    // without room for the 6-bit copy, many rows take the fp16 route
+    const uint64_t fp6_bytes = slhip::quant_fp6_bytes(qformat, n, k, group_size, layout);
+    if (fp6_bytes != 0 && hipMalloc(reinterpret_cast<void**>(&pb.fp6), fp6_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        pb.fp6 = nullptr;
     }
     pb.desc.quantized = 1;
     pb.desc.qformat = qformat;
@@ -1692,6 +1705,8 @@ sl_status sl_hip_bind_quantized(sl_hip_device* d, uint32_t payload, uint32_t sca
     pb.layout = layout;
     hipError_t e = slhip::launch_quant_repack(static_cast<const uint8_t*>(pb.ptr), pb.tiles, qformat, n, k, layout,
                                               d->stream);
+    if (e == hipSuccess && pb.fp6)
+        e = slhip::launch_fp6_repack(static_cast<const uint8_t*>(pb.ptr), pb.fp6, n, k, d->stream);
     if (e == hipSuccess && pb.tile_scales)
         e = slhip::launch_scale_repack(static_cast<const float*>(d->buffers[scales].ptr), pb.tile_scales, n, k,
                                        group_size, d->stream);

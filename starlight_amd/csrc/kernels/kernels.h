@@ -35,6 +35,7 @@ hipError_t load_code_gemv_dense();
 hipError_t load_code_layout();
 hipError_t load_code_matmul();
 hipError_t load_code_norm_softmax();
+hipError_t load_code_qgemm_fp6();
 hipError_t load_code_qgemm_mfma();
 hipError_t load_code_qgemv_fused();
 hipError_t load_code_qgemv_mfma();
@@ -44,7 +45,7 @@ inline hipError_t preload_code() {
     hipError_t (*const loads[])() = {load_code_attention, load_code_elementwise, load_code_layout,
                                      load_code_matmul,    load_code_norm_softmax, load_code_qgemm_mfma,
                                      load_code_qgemv_fused, load_code_qgemv_mfma, load_code_qmatmul,
-                                     load_code_rope,      load_code_gemv_dense};
+                                     load_code_rope,      load_code_gemv_dense, load_code_qgemm_fp6};
     hipError_t first = hipSuccess;
     for (auto load : loads) {
         const hipError_t e = load();
@@ -210,6 +211,7 @@ struct QuantWeight {
     uint64_t n, k;
     QuantLayout layout;
     const float* tile_scales;  // Mfma: scales in wave order (quant_tile_scale_floats), else null
+    const uint8_t* fp6;        // INT4 with groups of whole superblocks: 6-bit copy (quant_fp6_bytes), or null
 };
 QuantLayout quant_layout_for(uint32_t format, uint64_t n, uint64_t k, uint32_t group);
 uint64_t quant_tile_bytes(uint32_t format, uint64_t n, uint64_t k, QuantLayout layout);
@@ -222,6 +224,10 @@ hipError_t launch_quant_repack(const uint8_t* payload, uint8_t* tiles, uint32_t 
 uint64_t quant_tile_scale_floats(uint64_t n, uint64_t k, uint32_t group, QuantLayout layout);
 hipError_t launch_scale_repack(const float* scales, float* tile_scales, uint64_t n, uint64_t k, uint32_t group,
                                hipStream_t s);
+// INT4 codes as 6-bit floats in matrix-core operand order, the copy the
+// many-row q-GEMM reads (qgemm_fp6.hip); 0 bytes where it takes no such weight.
+uint64_t quant_fp6_bytes(uint32_t format, uint64_t n, uint64_t k, uint32_t group, QuantLayout layout);
+hipError_t launch_fp6_repack(const uint8_t* payload, uint8_t* tiles, uint64_t n, uint64_t k, hipStream_t s);
 // out[m, n] = sum_k a[m, k] * dequant(w)[n, k]  (a: [m, k] row-major)
 // m > 16 on the Mfma layout (k % 128 == 0): fp16 matrix cores on activations
 // split into two fp16 parts per element; hipErrorNotSupported when the
@@ -244,6 +250,12 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
                               uint64_t m, const Workspace& ws, hipStream_t s, const float* u = nullptr,
                               const float* const* resid = nullptr, float* const* out2 = nullptr,
                               const float* gamma = nullptr, float eps = 0.f);
+// The route of launch_qgemm_multi for weights that all have a 6-bit copy
+// (the same arguments; hipErrorNotSupported, nothing launched, otherwise).
+bool qgemm_fp6_takes(const float* a, const QuantWeight* const* w, uint32_t nseg, uint64_t m, const Workspace& ws);
+hipError_t launch_qgemm_fp6(const float* a, const QuantWeight* const* w, float* const* out, uint32_t nseg, uint64_t m,
+                            const Workspace& ws, hipStream_t s, const float* u, const float* const* resid,
+                            float* const* out2, const float* gamma, float eps);
 hipError_t launch_qmatmul(const float* a, const QuantWeight& w, float* out, uint64_t m, const Workspace& ws,
                           hipStream_t s);
 // The MFMA decode path (m <= 16, Mfma layout); returns hipErrorNotSupported

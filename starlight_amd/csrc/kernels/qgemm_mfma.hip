@@ -30,6 +30,7 @@
 //    (codes8: through the mantissa of 1024, no converts).
 #include "common.h"
 #include "kernels.h"
+#include "qgemm_act.h"
 #include "starlight_hip.h"
 
 #include <type_traits>
@@ -48,21 +49,6 @@ constexpr int kStepK = 32;     // k per MFMA step (an LDS stage holds KS = 32 or
 template <int KS>
 constexpr int row_pad() { return KS == 32 ? 48 : 72; }
 constexpr int kExpBias = 15;   // scaled rows stay below 2^15
-
-// The activation element: a, or with a second input u (SwiGlu's down
-// projection) silu(a) * u, the elementwise kernels' formula
-// (elementwise.rs:10-12): (a * (1 / (1 + exp(-a)))) * u.
-__device__ __forceinline__ float4 act4(const float4* row, const float4* urow, uint32_t i) {
-    float4 v = row[i];
-    if (urow != nullptr) {
-        const float4 u = urow[i];
-        v.x = (v.x * (1.0f / (1.0f + expf(-v.x)))) * u.x;
-        v.y = (v.y * (1.0f / (1.0f + expf(-v.y)))) * u.y;
-        v.z = (v.z * (1.0f / (1.0f + expf(-v.z)))) * u.z;
-        v.w = (v.w * (1.0f / (1.0f + expf(-v.w)))) * u.w;
-    }
-    return v;
-}
 
 // Within every aligned group of 8 along k, position j of the split
 // activations and of the converted codes holds element kPerm8[j]: the order
@@ -535,6 +521,10 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
     if (!qgemm_mfma_takes(a, w, nseg, m, ws)) return hipErrorNotSupported;
     const QuantWeight& w0 = *w[0];
     if (gamma != nullptr && (u != nullptr || !qgemm_norm_takes(w0.k, gamma))) return hipErrorNotSupported;
+    {
+        const hipError_t e6 = launch_qgemm_fp6(a, w, out, nseg, m, ws, s, u, resid, out2, gamma, eps);
+        if (e6 != hipErrorNotSupported) return e6;
+    }
     const SplitLayout lay = split_layout(m, w0.k);
     _Float16* hi = reinterpret_cast<_Float16*>(ws.data);
     _Float16* lo = reinterpret_cast<_Float16*>(ws.data + lay.lo_at);

@@ -1,0 +1,139 @@
+"""INT4 q-GEMM for many rows on the 6-bit matrix cores, against float64.
+
+Bound: a superblock of 128 k is five products summed in f32 (each within 2^-22
+of the magnitudes it adds) and one multiply-add, superblocks add in f32, and
+an activation keeps 24 bits below the largest of the 32 that share its
+exponent (here: of its superblock's 128).
+"""
+import numpy as np
+import pytest
+
+from starlight_amd import quant
+from starlight_amd.ir import BufferRef, Op, QuantFormat, Value, ValueRole
+
+pytestmark = pytest.mark.gpu
+
+
+def weight(hip, n, k, group, r, codes=None):
+    """(ref, value, float64 weight) of a bound INT4 weight with codes -8..7."""
+    if codes is None:
+        codes = r.integers(-8, 8, (n, k)).astype(np.int8)
+    scales = r.uniform(0.001, 0.05, (n, k // group)).astype(np.float32)
+    words = quant.pack_codes(codes, QuantFormat.INT4)
+    pb, sb = hip.upload_new_u32(words), hip.upload_new_f32(scales.ravel())
+    hip.bind_quantized(pb, sb, QuantFormat.INT4, group, n, k)
+    deq = codes.astype(np.float64) * np.repeat(scales.astype(np.float64), group, axis=1)
+    return BufferRef(pb, 0, words.size), Value.quantized([n, k], QuantFormat.INT4, group), deq
+
+
+def run(hip, a, w):
+    m, k = a.shape
+    wr, wv, deq = w
+    n = deq.shape[0]
+    out = hip.allocate_f32(m * n, 256)
+    hip.upload_f32(out, np.full(m * n, 7.0, np.float32))
+    ab = hip.upload_new_f32(a)
+    hip.dispatch(Op.matmul_nt(), [BufferRef(ab, 0, m * k), wr], [Value.f32([m, k]), wv], [BufferRef(out, 0, m * n)],
+                 [Value.f32([m, n])])
+    return hip.read_f32(out, m * n).reshape(m, n)
+
+
+def assert_products(got, a, deq):
+    a64 = a.astype(np.float64)
+    m, k = a.shape
+    top = np.repeat(np.abs(a64).reshape(m, k // 128, 128).max(axis=2), 128, axis=1)
+    bound = (k / 128 + 8) * 2.0**-22 * (np.abs(a64) @ np.abs(deq).T) + 2.0**-25 * (top @ np.abs(deq).T)
+    diff = np.abs(got.astype(np.float64) - a64 @ deq.T)
+    assert np.all(diff <= bound + 1e-37), float(np.max(diff - bound))
+
+
+# m, n around the tiles' edges (32, 64, 128 rows; 128, 256 columns); k of one
+# superblock, with and without slices, rows held in 1, 2 and 4 units per
+# thread (4096, 8192, 16384) and past them
+@pytest.mark.parametrize("m,n,k,group", [
+    (17, 1, 128, 128), (31, 15, 256, 128), (33, 127, 384, 128), (64, 129, 1152, 128), (65, 260, 4096, 4096),
+    (100, 48, 4224, 128), (129, 16, 8320, 128), (20, 33, 16384, 256), (40, 50, 16512, 128), (300, 520, 512, 256),
+    (257, 2050, 640, 128), (520, 4100, 256, 128), (1030, 3000, 384, 128)])
+def test_products(hip, m, n, k, group):
+    r = np.random.default_rng(m + n + k)
+    a = (r.standard_normal((m, k)) * 10.0 ** r.uniform(-6, 3, (m, 1))).astype(np.float32)
+    a[3] = 0.0
+    w = weight(hip, n, k, group, r)
+    got = run(hip, a, w)
+    assert np.all(got[3] == 0.0)
+    assert_products(got, a, w[2])
+
+
+def test_elements_far_below_their_row_keep_their_bits(hip):
+    """Blocks of a row 2^40 below its maximum are cut at their own exponent:
+    with zero codes under the large blocks, the small ones' products remain."""
+    r = np.random.default_rng(4)
+    m, n, k = 48, 64, 512
+    a = r.standard_normal((m, k)).astype(np.float32)
+    a[:, :128] *= np.float32(2.0**40)
+    codes = r.integers(-8, 8, (n, k)).astype(np.int8)
+    codes[:, :128] = 0
+    w = weight(hip, n, k, 128, r, codes)
+    got = run(hip, a, w)
+    assert_products(got, a[:, 128:], w[2][:, 128:])
+
+
+@pytest.mark.parametrize("scale", [1e-42, 1e-37, 1e30, 3e37])
+def test_extreme_magnitudes(hip, scale):
+    r = np.random.default_rng(9)
+    a = (r.uniform(-1, 1, (20, 256)) * scale).astype(np.float32)
+    w = weight(hip, 40, 256, 128, r)
+    got = run(hip, a, w)
+    want = a.astype(np.float64) @ w[2].T
+    finite = np.abs(want) < 3.4e38
+    err = np.abs(got.astype(np.float64) - want)[finite]
+    assert np.all(err <= 1e-5 * np.sqrt(256) * 8 * 0.05 * scale + 2e-45)
+
+
+def test_infinities_and_nan_stay_in_their_row(hip):
+    r = np.random.default_rng(6)
+    a = r.standard_normal((40, 384)).astype(np.float32)
+    a[5, 100], a[17, 383], a[30, 0] = np.inf, np.nan, -np.inf
+    w = weight(hip, 70, 384, 128, r)
+    got = run(hip, a, w)
+    bad = [5, 17, 30]
+    assert np.all(np.isnan(got[bad]))
+    keep = [i for i in range(40) if i not in bad]
+    assert_products(got[keep], a[keep], w[2])
+
+
+def test_reuploaded_payload_and_scales_refresh_the_copy(hip):
+    r = np.random.default_rng(8)
+    n, k = 48, 256
+    a = r.standard_normal((24, k)).astype(np.float32)
+    w = weight(hip, n, k, 128, r)
+    run(hip, a, w)
+    codes = r.integers(-8, 8, (n, k)).astype(np.int8)
+    hip.upload_u32(w[0].buffer, quant.pack_codes(codes, QuantFormat.INT4))
+    scales = r.uniform(0.001, 0.05, (n, 2)).astype(np.float32)
+    hip.upload_f32(w[0].buffer + 1, scales.ravel())
+    deq = codes.astype(np.float64) * np.repeat(scales.astype(np.float64), 128, axis=1)
+    assert_products(run(hip, a, (w[0], w[1], deq)), a, deq)
+
+
+@pytest.mark.parametrize("rows,k,ns", [(20, 2048, (64, 32, 32)), (77, 4096, (300, 129, 65)), (140, 512, (256, 16, 48))])
+def test_norm_and_three_projections_in_slices(hip, rows, k, ns):
+    """One launch for three weights, its k slices' sums added per weight."""
+    r = np.random.default_rng(rows)
+    x = r.standard_normal((rows, k)).astype(np.float32)
+    g = r.uniform(0.5, 1.5, k).astype(np.float32)
+    xb, gb = hip.upload_new_f32(x), hip.upload_new_f32(g)
+    ws = [weight(hip, n, k, 128, r) for n in ns]
+    normed = BufferRef(hip.allocate_f32(rows * k, 256), 0, rows * k)
+    outs = [BufferRef(hip.allocate_f32(rows * n, 256), 0, rows * n) for n in ns]
+    act = Value.f32([rows, k])
+    before = hip.stats()["fused_commands"]
+    hip.dispatch(Op.rms_norm(1e-5), [BufferRef(xb, 0, rows * k), BufferRef(gb, 0, k)],
+                 [act, Value.f32([k], ValueRole.PARAM)], [normed], [act])
+    for (wr, wv, _), out, n in zip(ws, outs, ns):
+        hip.dispatch(Op.matmul_nt(), [normed, wr], [act, wv], [out], [Value.f32([rows, n])])
+    hip.synchronize()
+    assert hip.stats()["fused_commands"] - before == 4
+    a = hip.read_f32(normed.buffer, rows * k).reshape(rows, k)
+    for (_, _, deq), out, n in zip(ws, outs, ns):
+        assert_products(hip.read_f32(out.buffer, rows * n).reshape(rows, n), a, deq)
