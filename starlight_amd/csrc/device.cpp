@@ -306,7 +306,7 @@ hipError_t launch(Device* d, const Plan& p, const sl_buffer_ref* in, const sl_bu
                                       p.batch * p.m, ws, s);
             }
             return launch_matmul(fptr(d, in[0]), fptr(d, in[1]), fptr(d, out[0]), p.batch, p.batch_a, p.batch_b,
-                                 p.m, p.k, p.n, p.code == SL_OP_MATMUL_NT, s);
+                                 p.m, p.k, p.n, p.code == SL_OP_MATMUL_NT, ws, s);
         }
         case SL_OP_SOFTMAX:
             return launch_softmax(fptr(d, in[0]), fptr(d, out[0]), p.rows, p.cols, false, 0, 0, nullptr, s);
@@ -765,10 +765,10 @@ size_t try_fuse(Device* d, size_t i, hipError_t* err) {
     return 0;
 }
 
-// The same units on dense f32 weights, for at most 32 rows (decode):
-// [RmsNorm +] up to three MatMulNT reading the same rows, or one MatMulNT +
-// the residual Add, or [RmsNorm +] SwiGlu [+ the residual Add], as one dense
-// GEMV launch each (two for SwiGlu). Blocks of a launch write outputs while
+// The same units on dense f32 weights: [RmsNorm +] up to three MatMulNT
+// reading the same rows, or one MatMulNT + the residual Add, or, for at most
+// 32 rows (decode), [RmsNorm +] SwiGlu [+ the residual Add], as one dense
+// GEMV or GEMM launch each (two for SwiGlu). Blocks of a launch write outputs while
 // others still read the weights, so no output may overlap a weight of the
 // launch either. Returns the commands covered (0: nothing launched).
 size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
@@ -799,14 +799,17 @@ size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
         f.normed = fptr(d, norm->out);
         f.eps = norm->plan.eps;
     }
-    // the norm inside the GEMV's prologue, or ahead of it on its own
+    // the norm inside the GEMV's prologue, or ahead of the launch on its own
     const auto run = [&]() -> hipError_t {
-        if (!norm || gemv_dense_norm_takes(f)) return launch_gemv_dense(f, d->stream);
-        const hipError_t e = launch_rms_norm(f.a, f.gamma, f.normed, f.m, f.k, f.eps, d->stream);
-        if (e != hipSuccess) return e;
-        f.a = f.normed;
-        f.gamma = nullptr;
-        return launch_gemv_dense(f, d->stream);
+        if (norm && !gemv_dense_norm_takes(f)) {
+            const hipError_t e = launch_rms_norm(f.a, f.gamma, f.normed, f.m, f.k, f.eps, d->stream);
+            if (e != hipSuccess) return e;
+            f.a = f.normed;
+            f.gamma = nullptr;
+        }
+        const hipError_t e = launch_gemv_dense(f, d->stream);
+        return e == hipErrorNotSupported ? launch_gemm_dense(f, Workspace{d->workspace, d->workspace_floats}, d->stream)
+                                         : e;
     };
 
     if (c1.plan.code == SL_OP_MATMUL_NT && !c1.plan.quant[1].present) {
@@ -845,7 +848,10 @@ size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
                 ++used;
             }
         }
-        if (used == 1 || !gemv_dense_takes(f)) return 0;
+        GemvDense plain = f;  // as the GEMM would be given it
+        plain.gamma = nullptr;
+        if (norm) plain.a = f.normed;
+        if (used == 1 || !(gemv_dense_takes(f) || gemm_dense_takes(plain))) return 0;
         *err = run();
         d->stats.fused_commands += used;
         return used;

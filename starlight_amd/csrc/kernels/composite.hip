@@ -17,7 +17,7 @@ namespace slhip {
 hipError_t launch_linear(const float* a, const WeightRef& w, float* out, uint64_t rows, uint64_t n,
                          uint64_t k, const Workspace& ws, hipStream_t s) {
     if (w.quantized()) return launch_qmatmul(a, w.quant, out, rows, ws, s);
-    return launch_matmul(a, w.dense, out, 1, 1, 1, rows, k, n, true, s);
+    return launch_matmul(a, w.dense, out, 1, 1, 1, rows, k, n, true, ws, s);
 }
 
 // Rows per chunk of launch_swiglu with a workspace of ws_floats: its g and
@@ -82,8 +82,25 @@ hipError_t launch_swiglu(const float* x, const WeightRef& gate, const WeightRef&
         } else {
             // (never with gamma: the check above covers every chunk)
             if (gamma != nullptr) return hipErrorInvalidValue;
-            e = launch_linear(xr, gate, g, rc, inter, hidden, rest, s);
-            if (e == hipSuccess) e = launch_linear(xr, up, u, rc, inter, hidden, rest, s);
+            e = hipErrorNotSupported;
+            if (!gate.quantized() && !up.quantized() && rc > 32) {
+                GemvDense f{};
+                f.a = xr;
+                f.nseg = 2;
+                f.m = rc;
+                f.k = hidden;
+                f.epilogue = kFusedPlain;
+                for (int t = 0; t < 2; ++t) {
+                    f.w[t] = t == 0 ? gate.dense : up.dense;
+                    f.n[t] = inter;
+                    f.out[t] = gu_out[t];
+                }
+                e = launch_gemm_dense(f, rest, s);
+            }
+            if (e == hipErrorNotSupported) {
+                e = launch_linear(xr, gate, g, rc, inter, hidden, rest, s);
+                if (e == hipSuccess) e = launch_linear(xr, up, u, rc, inter, hidden, rest, s);
+            }
         }
         if (e != hipSuccess) return e;
         float* const out_r = out + r0 * hidden;

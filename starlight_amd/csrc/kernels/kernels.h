@@ -31,6 +31,7 @@ struct Workspace {
 // them all and returns the first error.
 hipError_t load_code_attention();
 hipError_t load_code_elementwise();
+hipError_t load_code_gemm_dense();
 hipError_t load_code_gemv_dense();
 hipError_t load_code_layout();
 hipError_t load_code_matmul();
@@ -41,11 +42,13 @@ hipError_t load_code_qgemv_fused();
 hipError_t load_code_qgemv_mfma();
 hipError_t load_code_qmatmul();
 hipError_t load_code_rope();
+hipError_t load_code_slices();
 inline hipError_t preload_code() {
     hipError_t (*const loads[])() = {load_code_attention, load_code_elementwise, load_code_layout,
                                      load_code_matmul,    load_code_norm_softmax, load_code_qgemm_mfma,
                                      load_code_qgemv_fused, load_code_qgemv_mfma, load_code_qmatmul,
-                                     load_code_rope,      load_code_gemv_dense, load_code_qgemm_fp6};
+                                     load_code_rope,      load_code_gemv_dense, load_code_qgemm_fp6,
+                                     load_code_gemm_dense, load_code_slices};
     hipError_t first = hipSuccess;
     for (auto load : loads) {
         const hipError_t e = load();
@@ -196,7 +199,26 @@ uint64_t paged_attention_workspace_floats(const PagedAttentionArgs& p);
 // ---- dense f32 matmul (reference/matmul.rs) ----
 // out[b] = a[b or 0] x op(b[b or 0]); op = transpose when `nt`.
 hipError_t launch_matmul(const float* a, const float* b, float* out, uint64_t batch, uint64_t batch_a,
-                         uint64_t batch_b, uint64_t m, uint64_t k, uint64_t n, bool nt, hipStream_t s);
+                         uint64_t batch_b, uint64_t m, uint64_t k, uint64_t n, bool nt, const Workspace& ws,
+                         hipStream_t s);
+
+// ---- k slices of a GEMM (slices.hip) ----
+// Up to three outputs [m, n], unused ones with n == 0; slice z's partial sums
+// at partial + z slice_floats, the outputs one after the other. out = the
+// slices' sum; with out2, out2 = resid + out, and out may then be null.
+struct SliceSeg {
+    uint64_t n;
+    float* out;
+    const float* resid;
+    float* out2;
+};
+struct SliceSum {
+    const float* partial;
+    uint64_t slice_floats, m;
+    uint32_t slices;
+    SliceSeg seg[3];
+};
+hipError_t launch_slices_sum(const SliceSum& p, hipStream_t s);
 
 // ---- group-quantized weights (device-private layouts, see qmatmul.hip) ----
 enum class QuantLayout : uint32_t {
@@ -316,6 +338,10 @@ struct GemvDense {
 bool gemv_dense_takes(const GemvDense& f);
 bool gemv_dense_norm_takes(const GemvDense& f);
 hipError_t launch_gemv_dense(const GemvDense& f, hipStream_t s);
+// The same for any number of rows (gemm_dense.hip), no norm and no pair: needs
+// k % 4 == 0 and 16-byte aligned a and weights; k slices' sums go to ws.
+bool gemm_dense_takes(const GemvDense& f);
+hipError_t launch_gemm_dense(const GemvDense& f, const Workspace& ws, hipStream_t s);
 
 // Weights are dense f32 (pointer) or quantized (QuantWeight with tiles != null).
 struct WeightRef {

@@ -449,28 +449,6 @@ __global__ __launch_bounds__(kWave* WM* WN) void qgemm_fp6(Fp6Args p) {
         }
 }
 
-// Adds the slices' sums in slice order, with the residual Add where a weight
-// has one. V: elements per thread and step (4 where every n is a multiple of
-// four and the pointers allow it). Bound by the partial sums' reads.
-template <int V>
-__global__ __launch_bounds__(256) void fp6_slices_sum(Fp6Args p) {
-    typedef float vec __attribute__((ext_vector_type(V)));
-    const uint64_t step = static_cast<uint64_t>(gridDim.x) * 256 * V;
-    const uint64_t end0 = static_cast<uint64_t>(p.m) * p.seg[0].n;
-    const uint64_t end1 = end0 + static_cast<uint64_t>(p.m) * p.seg[1].n;
-    for (uint64_t i = (static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x) * V; i < p.slice_floats; i += step) {
-        vec v = *reinterpret_cast<const vec*>(p.partial + i);
-        for (uint32_t z = 1; z < p.slices; ++z) v += *reinterpret_cast<const vec*>(p.partial + z * p.slice_floats + i);
-        const int si = i < end0 ? 0 : i < end1 ? 1 : 2;
-        const uint64_t o = i - (si == 0 ? 0 : si == 1 ? end0 : end1);
-        float* const out = si == 0 ? p.seg[0].out : si == 1 ? p.seg[1].out : p.seg[2].out;
-        float* const out2 = si == 0 ? p.seg[0].out2 : si == 1 ? p.seg[1].out2 : p.seg[2].out2;
-        const float* const resid = si == 0 ? p.seg[0].resid : si == 1 ? p.seg[1].resid : p.seg[2].resid;
-        if (out != nullptr) *reinterpret_cast<vec*>(out + o) = v;
-        if (out2 != nullptr) *reinterpret_cast<vec*>(out2 + o) = *reinterpret_cast<const vec*>(resid + o) + v;
-    }
-}
-
 struct RecordLayout {
     uint64_t exp_at, floats;
 };
@@ -591,14 +569,11 @@ hipError_t launch_qgemm_fp6(const float* a, const QuantWeight* const* w, float* 
     p.m = static_cast<uint32_t>(m);
     p.sb_total = kk / 128;
     uint64_t n_total = 0;
-    bool quads = true;
     for (uint32_t i = 0; i < nseg; ++i) {
         const bool res = resid != nullptr && out2 != nullptr && out2[i] != nullptr;
         p.seg[i] = Fp6Seg{w[i]->fp6, w[i]->tile_scales, out[i], res ? resid[i] : nullptr, res ? out2[i] : nullptr,
                           static_cast<uint32_t>(w[i]->n), 0u};
         n_total += w[i]->n;
-        quads = quads && w[i]->n % 4 == 0 && aligned16(p.seg[i].out) && aligned16(p.seg[i].resid) &&
-                aligned16(p.seg[i].out2);
     }
     const uint64_t part_at = (lay.floats + 63) / 64 * 64;
     size_t shape = 0;
@@ -610,9 +585,14 @@ hipError_t launch_qgemm_fp6(const float* a, const QuantWeight* const* w, float* 
     else if (shape == 2) e = run_gemm<2, 4, 1, 4>(p, s);
     else e = run_gemm<2, 2, 1, 4>(p, s);
     if (e != hipSuccess || p.slices == 1) return e;
-    if (quads) fp6_slices_sum<4><<<grid_for(p.slice_floats / 4, 256, 8192), 256, 0, s>>>(p);
-    else fp6_slices_sum<1><<<grid_for(p.slice_floats, 256, 8192), 256, 0, s>>>(p);
-    return hipGetLastError();
+    SliceSum sum{};
+    sum.partial = p.partial;
+    sum.slice_floats = p.slice_floats;
+    sum.m = m;
+    sum.slices = p.slices;
+    for (uint32_t i = 0; i < nseg; ++i)
+        sum.seg[i] = SliceSeg{w[i]->n, p.seg[i].out, p.seg[i].resid, p.seg[i].out2};
+    return launch_slices_sum(sum, s);
 }
 
 // Loads this file's code object now: HIP loads one at the first use of

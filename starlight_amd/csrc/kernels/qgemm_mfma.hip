@@ -23,7 +23,7 @@
 //  * qgemm_mfma: 128 x 128 output tiles, 4 waves of 64 x 64 (4 x 4 MFMA
 //    tiles of 16 x 16), k in stages of 32 through double-buffered LDS; or
 //    64 x 128 tiles (waves of 32 x 64) in stages of 32 or 64; a grid z of
-//    2 cuts k in two slices whose partial sums gemm_slices_sum adds. The
+//    2 cuts k in two slices whose partial sums slices_sum adds. The
 //    weight stage is read from the tile layout (per 16-row tile and 128-k
 //    superblock; a 32-k stage is half of one 64-k half: 32 lanes x 8 bytes
 //    for INT4, x 16 bytes for INT8) and converted to fp16 codes in LDS
@@ -163,20 +163,6 @@ __global__ __launch_bounds__(256) void split_rows(const float* __restrict__ a, c
         }
     } else {
         for (uint32_t i = threadIdx.x; i < groups; i += 256) put8(i, act4(row, urow, 2 * i), act4(row, urow, 2 * i + 1));
-    }
-}
-
-// out[i] = the k slices' partial sums of element i, added in slice order;
-// with resid, out2[i] = resid[i] + out[i] (the residual Add's order), and
-// out may then be null (the sum itself not written).
-__global__ __launch_bounds__(256) void gemm_slices_sum(const float* __restrict__ partial, uint32_t slices,
-                                                       uint64_t count, float* out, const float* resid, float* out2) {
-    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x; i < count;
-         i += static_cast<uint64_t>(gridDim.x) * 256) {
-        float v = partial[i];
-        for (uint32_t z = 1; z < slices; ++z) v += partial[z * count + i];
-        if (out != nullptr) out[i] = v;
-        if (out2 != nullptr) out2[i] = resid[i] + v;
     }
 }
 
@@ -596,9 +582,13 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
         e = hipGetLastError();
         if (e != hipSuccess) return e;
         const bool res = resid != nullptr && out2 != nullptr && out2[0] != nullptr;
-        const uint64_t count = m * w0.n;
-        gemm_slices_sum<<<grid_for(count, 256, 4096), 256, 0, s>>>(p.partial, 2, count, out[0],
-                                                                  res ? resid[0] : nullptr, res ? out2[0] : nullptr);
+        SliceSum sum{};
+        sum.partial = p.partial;
+        sum.slice_floats = m * w0.n;
+        sum.m = m;
+        sum.slices = 2;
+        sum.seg[0] = SliceSeg{w0.n, out[0], res ? resid[0] : nullptr, res ? out2[0] : nullptr};
+        return launch_slices_sum(sum, s);
     }
     return hipGetLastError();
 }
