@@ -50,6 +50,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "qgemm_act.h"
+#include "qgemm_plan.h"
 #include "starlight_hip.h"
 
 namespace slhip {
@@ -470,51 +471,18 @@ hipError_t run_gemm(Fp6Args& p, hipStream_t s) {
     return hipGetLastError();
 }
 
-// A block shape: its tile, the blocks a CU holds at once, and the time of one
-// superblock pass (us, MI355X) of 1, 2, ... blocks on a CU together. Measured
-// with [28672 x 4096], [4096 x 14336] and [4096 x 4096] at M = 20 to 1024.
-// Larger tiles read the activations' digits and the weights less often per
-// product (0.74 us per 32 x 256 outputs in 128 x 256 tiles, 0.81, 0.86 and
+// Measured with [28672 x 4096], [4096 x 14336] and [4096 x 4096] at M = 20 to
+// 1024. Larger tiles read the activations' digits and the weights less often
+// per product (0.74 us per 32 x 256 outputs in 128 x 256 tiles, 0.81, 0.86 and
 // 1.04 in the others); smaller ones reach every CU with fewer rows.
-struct Shape {
-    uint32_t bm, bn, most;
-    float pass[4];
-};
-constexpr Shape kShapes[] = {{128, 256, 1, {2.95f}},
-                             {64, 256, 2, {1.95f, 3.2f}},
-                             {32, 256, 2, {1.1f, 1.72f}},
-                             {32, 128, 4, {0.7f, 1.1f, 1.6f, 2.07f}}};
-
-// The shape and k slices with the least estimated time: each CU's blocks run
-// in rounds of as many as it holds, a pass per superblock of a slice; slices
-// add a launch (3.5 us) and the partial sums' traffic, written and read once
-// (4 TB/s). [4096 x 14336] at M = 77: 39 us in 32 x 128 tiles and 8 slices, 204
-// in 64 x 256 ones and one; at M = 1024 225 us in 64 x 256 and 4 slices, 201 in
-// 128 x 256 and 2; [4096 x 4096] at M = 512 48 us in 64 x 256 and 4 slices, 96
-// in 128 x 256 and one.
-void choose(const Fp6Args& p, uint64_t n_total, uint64_t room_floats, size_t* shape, uint32_t* slices) {
-    const uint32_t cus = compute_units();
-    float best = INFINITY;
-    for (size_t c = 0; c < sizeof(kShapes) / sizeof(kShapes[0]); ++c) {
-        const Shape& x = kShapes[c];
-        uint64_t tiles = 0;
-        for (uint32_t i = 0; i < p.nseg; ++i) tiles += (p.seg[i].n + x.bn - 1) / x.bn;
-        tiles *= (p.m + x.bm - 1) / x.bm;
-        for (uint32_t z = 1; z <= 8 && z <= p.sb_total; z *= 2) {
-            if (z > 1 && z * p.m * n_total > room_floats) break;
-            const uint64_t per_cu = (tiles * z + cus - 1) / cus;
-            const uint32_t rest = static_cast<uint32_t>(per_cu % x.most);
-            float t = static_cast<float>(per_cu / x.most) * x.pass[x.most - 1] + (rest ? x.pass[rest - 1] : 0.f);
-            t *= static_cast<float>((p.sb_total + z - 1) / z);
-            if (z > 1) t += 3.5f + static_cast<float>(p.m * n_total) * 4.f * static_cast<float>(2 * z + 1) / 4e6f;
-            if (t < best) {
-                best = t;
-                *shape = c;
-                *slices = z;
-            }
-        }
-    }
-}
+// [4096 x 14336] at M = 77: 39 us in 32 x 128 tiles and 8 slices, 204 in 64 x
+// 256 ones and one; at M = 1024 225 us in 64 x 256 and 4 slices, 201 in 128 x
+// 256 and 2; [4096 x 4096] at M = 512 48 us in 64 x 256 and 4 slices, 96 in 128
+// x 256 and one.
+constexpr GemmShape kShapes[] = {{128, 256, 1, {2.95f}},
+                                 {64, 256, 2, {1.95f, 3.2f}},
+                                 {32, 256, 2, {1.1f, 1.72f}},
+                                 {32, 128, 4, {0.7f, 1.1f, 1.6f, 2.07f}}};
 
 }  // namespace
 
@@ -568,16 +536,20 @@ hipError_t launch_qgemm_fp6(const float* a, const QuantWeight* const* w, float* 
     p.nseg = nseg;
     p.m = static_cast<uint32_t>(m);
     p.sb_total = kk / 128;
-    uint64_t n_total = 0;
+    uint64_t n_total = 0, n[kFusedMaxSegs] = {};
     for (uint32_t i = 0; i < nseg; ++i) {
         const bool res = resid != nullptr && out2 != nullptr && out2[i] != nullptr;
         p.seg[i] = Fp6Seg{w[i]->fp6, w[i]->tile_scales, out[i], res ? resid[i] : nullptr, res ? out2[i] : nullptr,
                           static_cast<uint32_t>(w[i]->n), 0u};
-        n_total += w[i]->n;
+        n[i] = w[i]->n;
+        n_total += n[i];
     }
     const uint64_t part_at = (lay.floats + 63) / 64 * 64;
-    size_t shape = 0;
-    choose(p, n_total, part_at < ws.floats ? ws.floats - part_at : 0, &shape, &p.slices);
+    const GemmChoice best =
+        choose_gemm(kShapes, n, nseg, m, p.sb_total, part_at < ws.floats ? ws.floats - part_at : 0,
+                    [](uint32_t) { return true; });
+    const size_t shape = best.shape;
+    p.slices = best.slices;
     p.partial = p.slices > 1 ? ws.data + part_at : nullptr;
     p.slice_floats = m * n_total;
     if (shape == 0) e = run_gemm<4, 4, 2, 4>(p, s);

@@ -31,6 +31,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "qgemm_act.h"
+#include "qgemm_plan.h"
 #include "starlight_hip.h"
 
 #include <type_traits>
@@ -192,9 +193,10 @@ struct GemmArgs {
     const int* row_exp;
     GemmSeg seg[kFusedMaxSegs];
     uint32_t nseg, m, k, group, groups, sb_total;
-    // k cut into gridDim.z slices of k / gridDim.z (one weight only): slice z
-    // writes its m x n partial sums at partial + z m n, added up afterwards
+    // k cut into gridDim.z slices of k / gridDim.z: slice z writes its partial
+    // sums at partial + z slice_floats, the weights' m x n one after the other
     float* partial;
+    uint64_t slice_floats;
 };
 
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
@@ -444,6 +446,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         }
     }
 
+    const uint64_t before = si == 0 ? 0 : p.seg[0].n + (si == 1 ? 0 : p.seg[1].n);  // columns of earlier weights
+    float* const part = gridDim.z > 1 ? p.partial + bz * p.slice_floats + before * p.m : nullptr;
     // lane holds rows 4 (lane / 16) + e of each row tile, column lane % 16
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -458,8 +462,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
                 if (col >= n) continue;
                 const uint64_t o = static_cast<uint64_t>(row) * n + col;
                 const float val = ldexpf(acc[i][j][e], sh);
-                if (gridDim.z > 1) {
-                    p.partial[static_cast<uint64_t>(bz) * p.m * n + o] = val;
+                if (part != nullptr) {
+                    part[o] = val;
                     continue;
                 }
                 if (out != nullptr) out[o] = val;
@@ -471,6 +475,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 }  // namespace
 
 namespace {
+
+// Measured with [28672 x 4096], [6144 x 4096], [4096 x 14336] and [4096 x 4096]
+// at M = 20 to 1024. With two slices at most, and those for one weight only,
+// INT8 [4096 x 14336] took 155 us at M = 77 (now 58, 64-row blocks and 8
+// slices), 159 at M = 200 (89) and 185 at M = 500 (170).
+constexpr GemmShape kShapes[] = {{128, 128, 2, {3.1f, 4.8f}}, {64, 128, 2, {1.95f, 3.0f}}};
 
 // hi and lo (fp16, m x k each), then the row exponents, in the workspace
 struct SplitLayout {
@@ -507,10 +517,9 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
     if (!qgemm_mfma_takes(a, w, nseg, m, ws)) return hipErrorNotSupported;
     const QuantWeight& w0 = *w[0];
     if (gamma != nullptr && (u != nullptr || !qgemm_norm_takes(w0.k, gamma))) return hipErrorNotSupported;
-    {
-        const hipError_t e6 = launch_qgemm_fp6(a, w, out, nseg, m, ws, s, u, resid, out2, gamma, eps);
-        if (e6 != hipErrorNotSupported) return e6;
-    }
+    // the 6-bit matrix cores where every weight has its 6-bit copy
+    hipError_t e = launch_qgemm_fp6(a, w, out, nseg, m, ws, s, u, resid, out2, gamma, eps);
+    if (e != hipErrorNotSupported) return e;
     const SplitLayout lay = split_layout(m, w0.k);
     _Float16* hi = reinterpret_cast<_Float16*>(ws.data);
     _Float16* lo = reinterpret_cast<_Float16*>(ws.data + lay.lo_at);
@@ -522,7 +531,7 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
     else if (w0.k <= 2048 * 8) split_rows<8><<<sgrid, 256, 0, s>>>(a, u, hi, lo, row_exp, kk, nullptr, 0.f);
     else if (w0.k <= 2048 * 16) split_rows<16><<<sgrid, 256, 0, s>>>(a, u, hi, lo, row_exp, kk, nullptr, 0.f);
     else split_rows<0><<<sgrid, 256, 0, s>>>(a, u, hi, lo, row_exp, kk, nullptr, 0.f);
-    hipError_t e = hipGetLastError();
+    e = hipGetLastError();
     if (e != hipSuccess) return e;
     GemmArgs p{};
     p.ahi = hi;
@@ -541,23 +550,24 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
     p.group = w0.group;
     p.groups = static_cast<uint32_t>(w0.k / w0.group);
     p.sb_total = static_cast<uint32_t>(w0.k / 128);
-    // 128-row blocks, or 64-row ones (three per CU, each with less operand
-    // reuse) when 128-row blocks would not give every CU one. Measured on
-    // MI355X: M = 1024 [4096 x 4096] (256 blocks of 128 rows) runs faster in
-    // 64-row blocks; M = 512 [14336 x 4096] (448) runs slower (200 -> 250 us).
-    // 128-row blocks, or when they would not give every CU one: k in two
-    // slices of 128-row blocks (one weight, the slice a whole number of
-    // groups and 128-k superblocks, room for the partial sums), else 64-row
-    // blocks. Measured on MI355X at M = 1024: [4096 x 14336] 395-402 us in
-    // k slices (the slice sums included) against 440 us in 64-row blocks.
-    const uint64_t blocks128 = static_cast<uint64_t>(blocks) * ((m + 127) / 128);
+    uint64_t n[kFusedMaxSegs] = {}, n_total = 0;
+    for (uint32_t i = 0; i < nseg; ++i) {
+        n[i] = w[i]->n;
+        n_total += n[i];
+    }
     const uint64_t part_at = (lay.floats + 63) / 64 * 64;
-    const bool sliced = blocks128 <= compute_units() && nseg == 1 && (w0.k / 2) % 128 == 0 &&
-                        (w0.k / 2) % w0.group == 0 && part_at + 2 * m * w0.n <= ws.floats;
-    const bool rows64 = blocks128 <= compute_units() && !sliced;
+    // 128-row blocks reuse each operand more; 64-row ones and k slices (whole
+    // groups and superblocks each) reach every CU with fewer rows.
+    const GemmChoice best = choose_gemm(kShapes, n, nseg, m, p.sb_total, part_at < ws.floats ? ws.floats - part_at : 0,
+                                        [&](uint32_t z) {
+                                            return z == 1 || (w0.k % (z * 128) == 0 && w0.k % (z * w0.group) == 0);
+                                        });
+    const bool rows64 = best.shape == 1;
+    const uint32_t slices = best.slices;
     const bool deep = rows64 && w0.group % 64 == 0;  // 64-k stages
-    p.partial = sliced ? ws.data + part_at : nullptr;
-    const dim3 grid(blocks, static_cast<unsigned>(rows64 ? (m + 63) / 64 : (m + 127) / 128), sliced ? 2u : 1u);
+    p.partial = slices > 1 ? ws.data + part_at : nullptr;
+    p.slice_floats = m * n_total;
+    const dim3 grid(blocks, static_cast<unsigned>(rows64 ? (m + 63) / 64 : (m + 127) / 128), slices);
     // stages per group when it is a compile-time form: 128 / KS for group 128
     // (4 or 2), 2 for group 64 in 32-k stages; 0 otherwise
     const int ks = deep ? 64 : 32;
@@ -578,16 +588,15 @@ hipError_t launch_qgemm_multi(const float* a, const QuantWeight* const* w, float
         else SL_QGEMM(8, 128, 32);
     }
 #undef SL_QGEMM
-    if (sliced) {
+    if (slices > 1) {
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        const bool res = resid != nullptr && out2 != nullptr && out2[0] != nullptr;
         SliceSum sum{};
         sum.partial = p.partial;
-        sum.slice_floats = m * w0.n;
+        sum.slice_floats = p.slice_floats;
         sum.m = m;
-        sum.slices = 2;
-        sum.seg[0] = SliceSeg{w0.n, out[0], res ? resid[0] : nullptr, res ? out2[0] : nullptr};
+        sum.slices = slices;
+        for (uint32_t i = 0; i < nseg; ++i) sum.seg[i] = SliceSeg{n[i], out[i], p.seg[i].resid, p.seg[i].out2};
         return launch_slices_sum(sum, s);
     }
     return hipGetLastError();
