@@ -1028,9 +1028,22 @@ size_t try_fuse_attention(Device* d, size_t i, hipError_t* err) {
     // the mirror fits; otherwise it runs on its own and reads MergeHeads'
     // output, which must then be written.
     const Logged* mm = mh && i + used < n ? &d->log[i + used] : nullptr;
+    GemvDense dense{};  // the same for a dense weight
+    if (mm && mm->plan.code == SL_OP_MATMUL_NT && !mm->plan.quant[1].present && mm->plan.batch_b == 1 &&
+        mm->plan.batch_a == mm->plan.batch) {
+        dense.a = ws.data + mirror_at;
+        dense.w[0] = fptr(d, mm->in[1]);
+        dense.n[0] = mm->plan.n;
+        dense.out[0] = fptr(d, mm->out);
+        dense.nseg = 1;
+        dense.m = B * S;
+        dense.k = H * D;
+        dense.epilogue = kFusedPlain;
+    }
+    const bool dense_chain = gemv_dense_takes(dense);
     const bool chain = mm && mm->plan.code == SL_OP_MATMUL_NT && same_ref(mm->in[0], mh->out) &&
-                       mfma_weight(d, *mm, 1) && mm->plan.batch * mm->plan.m == B * S && mm->plan.k == H * D &&
-                       B * S <= 16 && mirror_at + B * S * H * D <= ws.floats;
+                       (mfma_weight(d, *mm, 1) || dense_chain) && mm->plan.batch * mm->plan.m == B * S &&
+                       mm->plan.k == H * D && B * S <= 16 && mirror_at + B * S * H * D <= ws.floats;
     const bool merged_needed = mh != nullptr && !dead_after(d, i + used, mh->out, chain ? i + used : SIZE_MAX);
     // outputs of the merge kernel: no overlap with the cache, or with each other
     if (overlaps(att, cache_ref) || (mh && overlaps(mh->out, cache_ref)) ||
@@ -1119,7 +1132,22 @@ size_t try_fuse_attention(Device* d, size_t i, hipError_t* err) {
         *err = e;
         return used;
     }
-    if (chain) {
+    if (chain && dense_chain) {
+        // (blocks write outputs while others still read the weight)
+        size_t extra = 1;
+        if (i + used + 1 < n) {
+            const Logged& ad = d->log[i + used + 1];
+            const int other = residual_port(ad, mm->out, B * S * dense.n[0], &mm->in[1], 1);
+            if (other >= 0) {
+                dense.epilogue = kFusedResidual;
+                dense.resid[0] = fptr(d, ad.in[other]);
+                dense.out2[0] = fptr(d, ad.out);
+                extra = 2;
+            }
+        }
+        e = launch_gemv_dense(dense, d->stream);
+        used += extra;
+    } else if (chain) {
         QuantWeight w = weight_ref(d, mm->in[1], mm->plan.quant[1]).quant;
         QgemvFused f{};
         f.a = a.mirror;
