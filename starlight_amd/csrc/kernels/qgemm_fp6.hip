@@ -24,15 +24,16 @@
 // Rate. Register-resident loops on MI355X reach 8.43 PFLOP/s with 6-bit
 // operands and 2.17 PFLOP/s with fp16 ones: five 6-bit products per multiply
 // allow 1.69 PFLOP/s of f32 result, two fp16 ones 1.08. With the split, against
-// the fp16 route: [28672 x 4096] M = 1024 399 us against 525 (602 TFLOP/s of
-// f32 result), M = 77 63 against 89; [4096 x 14336] M = 1024 227 against 304,
-// M = 512 126 against 186, M = 77 42 against 159; [4096 x 4096] M = 77 25
-// against 56. What bounds it now: a pass of a 64 x 256 tile needs about 1,300
-// cycles of products per SIMD, 1,200 of LDS and 900 of loads through the
-// vector cache (two tiles per CU: 2,600, 2,400 and 1,800 of about 6,000
-// measured); deeper operand prefetch and wave priorities changed nothing, and
-// gathering the records in operand order from memory (no LDS conflicts,
-// scattered 64-byte loads) was slower.
+// the fp16 route: [28672 x 4096] M = 1024 358 us against 525 (673 TFLOP/s of
+// f32 result), M = 77 58 against 89; [4096 x 14336] M = 1024 212 against 304,
+// M = 512 117 against 186, M = 77 41 against 159; [4096 x 4096] M = 77 24
+// against 56. What bounds it now: vector and matrix instructions of a SIMD's
+// waves do not overlap here, and a 64 x 256 tile's pass has 80 products (1,280
+// cycles) and about 160 vector instructions (640) per wave, two waves per
+// SIMD: 3,840 of about 6,000 cycles measured; LDS is busy a third of the time.
+// Deeper operand prefetch and wave priorities changed nothing, and gathering
+// the records in operand order from memory (no LDS conflicts, scattered
+// 64-byte loads) was slower.
 //
 // Kernels
 //  * repack_fp6 (bind): the codes as E2M3 in operand order, per 16-row tile
@@ -282,9 +283,20 @@ struct Fp6Args {
     uint64_t slice_floats;
 };
 
-// A block's waves are WM x WN, each 16 MT rows by 16 NT columns.
+// A load of 4, 8 or 16 bytes at a global address.
+template <typename T>
+__device__ __forceinline__ T load_at(__attribute__((address_space(1))) const uint8_t* p) {
+    typedef uint32_t words __attribute__((ext_vector_type(sizeof(T) / 4)));
+    const words v = *(__attribute__((address_space(1))) const words*)p;
+    return __builtin_bit_cast(T, v);
+}
+
+// A block's waves are WM x WN, each 16 MT rows by 16 NT columns. At most 256
+// registers a wave (two per SIMD): with more allowed, the compiler keeps the
+// digit sums in accumulation registers and moves each out before the vector
+// unit can add it, 128 moves in a 64 x 256 tile's pass (396 -> 360 us).
 template <int MT, int NT, int WM, int WN>
-__global__ __launch_bounds__(kWave* WM* WN) void qgemm_fp6(Fp6Args p) {
+__global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2))) void qgemm_fp6(Fp6Args p) {
     constexpr int T = kWave * WM * WN;
     constexpr uint32_t BM = 16 * MT * WM, BN = 16 * NT * WN;
     constexpr int NL = BM * 32 / T;  // 16-byte pieces of a stage per thread
@@ -316,11 +328,19 @@ __global__ __launch_bounds__(kWave* WM* WN) void qgemm_fp6(Fp6Args p) {
         uint2 hi[NT];
         float s[NT];
     };
-    uint32_t src[NL];  // this thread's 16-byte pieces: piece tid % 32 of rows tid / 32 + T / 32 i
+    uint32_t src[NL];  // byte offsets of this thread's pieces: piece tid % 32 of rows tid / 32 + T / 32 i
 #pragma unroll
     for (int i = 0; i < NL; ++i)
-        src[i] = min(m0 + tid / 32 + T / 32 * i, p.m - 1) * p.sb_total * (kRecord / 16) + tid % 32;
-    const uint4* const records = reinterpret_cast<const uint4*>(p.records);
+        src[i] = (min(m0 + tid / 32 + T / 32 * i, p.m - 1) * p.sb_total * (kRecord / 16) + tid % 32) * 16;
+    // A uniform base that stays in scalar registers plus a 32-bit lane offset
+    // per load: left to itself the compiler keeps one 64-bit vector address
+    // per load.
+    typedef __attribute__((address_space(1))) const uint8_t global_u8;
+    const auto scalar = [](const void* q) -> global_u8* {
+        global_u8* r = (global_u8*)q;
+        asm volatile("" : "+s"(r));
+        return r;
+    };
     const uint8_t* wt[NT];
     const float* ws[NT];
 #pragma unroll
@@ -329,19 +349,22 @@ __global__ __launch_bounds__(kWave* WM* WN) void qgemm_fp6(Fp6Args p) {
         wt[j] = SL_GSEG(tiles) + t * kTileBytes;
         ws[j] = SL_GSEG(scales) + t * 16;
     }
+    const uint32_t lane16 = lane * 16, lane8 = lane * 8, col4 = lane % 16 * 4;
     auto load_stage = [&](uint32_t sb) -> Stage {
         Stage r;
+        global_u8* const base = scalar(p.records + static_cast<uint64_t>(sb) * kRecord);
 #pragma unroll
-        for (int i = 0; i < NL; ++i) r.v[i] = records[static_cast<uint64_t>(src[i]) + sb * (kRecord / 16)];
+        for (int i = 0; i < NL; ++i) r.v[i] = load_at<uint4>(base + src[i]);
         return r;
     };
     auto load_weights = [&](uint32_t sb) -> Weights {
         Weights r;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            r.lo[j] = *reinterpret_cast<const uint4*>(wt[j] + sb * kTileBytes + lane * 16);
-            r.hi[j] = *reinterpret_cast<const uint2*>(wt[j] + sb * kTileBytes + 1024 + lane * 8);
-            r.s[j] = ws[j][sb * 16 + lane % 16];
+            global_u8* const base = scalar(wt[j] + static_cast<uint64_t>(sb) * kTileBytes);
+            r.lo[j] = load_at<uint4>(base + lane16);
+            r.hi[j] = load_at<uint2>(base + 1024 + lane8);
+            r.s[j] = load_at<float>(scalar(ws[j] + static_cast<uint64_t>(sb) * 16) + col4);
         }
         return r;
     };
@@ -370,10 +393,8 @@ __global__ __launch_bounds__(kWave* WM* WN) void qgemm_fp6(Fp6Args p) {
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    Weights w = load_weights(beg);
-    store_stage(0, load_stage(beg));
-    __syncthreads();
-    for (uint32_t sb = beg; sb < end; ++sb) {
+    // One superblock with weights w; returns the next one's.
+    auto pass = [&](uint32_t sb, const Weights w) -> Weights {
         const uint32_t buf = (sb - beg) & 1;
         // past the end the last superblock again: every pass issues the same loads
         const uint32_t nx = min(sb + 1, end - 1);
@@ -416,8 +437,18 @@ __global__ __launch_bounds__(kWave* WM* WN) void qgemm_fp6(Fp6Args p) {
         }
         store_stage(buf ^ 1, st);
         __syncthreads();
-        w = wx;
+        return wx;
+    };
+    Weights w0 = load_weights(beg);
+    store_stage(0, load_stage(beg));
+    __syncthreads();
+    // two passes per iteration: the weights' registers alternate, not moved
+    uint32_t sb = beg;
+    for (; sb + 1 < end; sb += 2) {
+        const Weights w1 = pass(sb, w0);
+        w0 = pass(sb + 1, w1);
     }
+    if (sb < end) pass(sb, w0);
 
     // accumulator value e of lane l: row 4 (l / 16) + e, column l % 16 of its
     // tile; (d / 8) (q / 8) 2^(E - Erow) 32^(j - 4) against d q 32^j 2^(E - 24)
@@ -480,7 +511,7 @@ hipError_t run_gemm(Fp6Args& p, hipStream_t s) {
 // 256 and 2; [4096 x 4096] at M = 512 48 us in 64 x 256 and 4 slices, 96 in 128
 // x 256 and one.
 constexpr GemmShape kShapes[] = {{128, 256, 1, {2.95f}},
-                                 {64, 256, 2, {1.95f, 3.2f}},
+                                 {64, 256, 2, {1.8f, 2.9f}},
                                  {32, 256, 2, {1.1f, 1.72f}},
                                  {32, 128, 4, {0.7f, 1.1f, 1.6f, 2.07f}}};
 
@@ -508,8 +539,8 @@ bool qgemm_fp6_takes(const float* a, const QuantWeight* const* w, uint32_t nseg,
             return false;
         n += x.n;
     }
-    // 16-byte pieces of the records in 32 bits
-    return m * (w[0]->k / 128) * (kRecord / 16) <= 0xffffffffull && m * n <= 0xffffffffffull &&
+    // byte offsets of the records in 32 bits
+    return m * (w[0]->k / 128) * kRecord <= 0xffffffffull && m * n <= 0xffffffffffull &&
            record_layout(m, w[0]->k).floats <= ws.floats;
 }
 
