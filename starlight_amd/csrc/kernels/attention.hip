@@ -954,7 +954,7 @@ __global__ __launch_bounds__(256 * KH) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // ---- prefill on the bf16 matrix cores ----
 //
-// The f32 matrix cores do 2,048 multiply-adds in 32 cycles, the bf16 ones 16,384
+// The f32 matrix cores do 1,024 multiply-adds in 32 cycles, the bf16 ones 8,192
 // in 16. A float is exactly three bf16 parts (8 + 8 + 8 significant bits),
 // x = h + m + l; of the nine products of two such splits the six down to 2^-16
 // (hh, hm, mh, hl, lh, mm) are kept, smallest first, so a product is off by
@@ -966,7 +966,7 @@ __global__ __launch_bounds__(256 * KH) __attribute__((amdgpu_waves_per_eu(2, 2))
 // per 16 dims, lane l holds dim l % 16 and the keys 4 (l / 16) .., 16 + 4 (l /
 // 16) .. - the keys whose weights the same lane holds after S^T), and
 // attn_prefill_bf16 copies tiles to LDS and reads them 16 bytes per lane,
-// without bank conflicts. The softmax is attn_prefill's; each product's sum
+// without bank conflicts. The softmax is attn_prefill's, in base 2; each product's sum
 // starts from zero and joins O^T with the rescale's multiply-add.
 //
 // Values whose parts or partial products could leave the range (NaN, infinity,
@@ -974,7 +974,7 @@ __global__ __launch_bounds__(256 * KH) __attribute__((amdgpu_waves_per_eu(2, 2))
 // in q per block; a block that sees one does its query tiles as attn_prefill.
 //
 // Per layer with the planes (f32 form before): 1024 rows, 32 heads of 128: 117 ->
-// 94 us; 3001 rows, 32 heads of 64: 519 -> 305; 2 x 256 rows after 256, heads of
+// 94 us; 3001 rows, 32 heads of 64: 519 -> 305; 2 x 256 rows after 640, heads of
 // 128: 146 -> 121. Bound by vector and matrix instructions (D = 128, per 32 keys
 // of a wave: 96 MFMA, 1,536 cycles, and about 300 vector instructions, 1,200) and,
 // with one block of 8 waves per CU at D = 128, the waits between them; D = 64 has
