@@ -966,8 +966,9 @@ __global__ __launch_bounds__(256 * KH) __attribute__((amdgpu_waves_per_eu(2, 2))
 // per 16 dims, lane l holds dim l % 16 and the keys 4 (l / 16) .., 16 + 4 (l /
 // 16) .. - the keys whose weights the same lane holds after S^T), and
 // attn_prefill_bf16 copies tiles to LDS and reads them 16 bytes per lane,
-// without bank conflicts. The softmax is attn_prefill's, in base 2; each product's sum
-// starts from zero and joins O^T with the rescale's multiply-add.
+// without bank conflicts. The softmax is attn_prefill's on unscaled scores, in base
+// 2 (so a negative scale, whose maximum is their minimum, is left to that form);
+// each product's sum starts from zero and joins O^T with the rescale's multiply-add.
 //
 // Values whose parts or partial products could leave the range (NaN, infinity,
 // 2^56 and above, below 2^-100) are found by attn_planes per tile (`flags`) and
@@ -1161,14 +1162,16 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void attn_prefill_bf16(
                 }
                 st[s2] = hi + lo;
             }
-            // exp(x scale) is exp2(x c), the product and the difference to
-            // the maximum rounded once; only a tile with keys past the
+            // exp(x scale - max(x scale)) is exp2((x - max(x)) c) for c >= 0:
+            // exactly 1 for the largest score, however large (a rounded x c
+            // differs from the exact one by more than 128 from 2^31 on, and
+            // its power of two overflows); only a tile with keys past the
             // wave's first query is masked (wave-uniform)
             const bool edge = kt + 32 > past + q0 + 1;
             float p[8];
             float tmax = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) p[i] = st[i / 4][i % 4] * c2;
+            for (int i = 0; i < 8; ++i) p[i] = st[i / 4][i % 4];
             if (edge) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
@@ -1181,10 +1184,10 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void attn_prefill_bf16(
             // A query can see none of the tile's keys (m_new == -inf): the
             // guards keep corr and every weight 0, not NaN.
             const float m_new = fmaxf(m, tmax);
-            const float corr = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+            const float corr = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - m_new) * c2);
             float psum = 0.f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(fmaf(st[i / 4][i % 4], c2, -m_new));
+            for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f((p[i] - m_new) * c2);
             if (edge) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
@@ -1227,8 +1230,8 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void attn_prefill_bf16(
         if (half == 1) continue;
         const float m1 = xs[x], l1 = xs[256 + x];
         const float mm = fmaxf(m, m1);
-        const float c0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mm);
-        const float c1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mm);
+        const float c0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mm) * c2);
+        const float c1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - mm) * c2);
         lsum = lsum * c0 + l1 * c1;
         if (t < g.seq) {
             const float inv = 1.0f / lsum;
@@ -1473,7 +1476,7 @@ hipError_t run_prefill(const AttentionArgs& a, const Geo& g, const Workspace& ws
     const uint64_t tiles = (a.max_seq + 63) / 64 * 2;  // an even count: stages are two tiles
     const uint64_t words = a.batch * a.kv_heads * tiles * (wide ? plane_words<128>() : plane_words<64>());
     const uint64_t flag_floats = (a.batch * a.kv_heads * tiles + 63) / 64 * 64, floats = flag_floats + 4 * words;
-    if (a.seq < (wide ? 256 : 512) || !(a.scale >= -32.f && a.scale <= 32.f) || tiles > 0xffffffull || keep + floats + 64 > ws.floats) {
+    if (a.seq < (wide ? 256 : 512) || !(a.scale >= 0.f && a.scale <= 32.f) || tiles > 0xffffffull || keep + floats + 64 > ws.floats) {
         if (wide) attn_prefill<128, 2><<<grid, 512, 0, s>>>(g, qtiles);
         else attn_prefill<64, 2><<<grid, 512, 0, s>>>(g, qtiles);
         return hipGetLastError();
