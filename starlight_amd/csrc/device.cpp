@@ -799,13 +799,22 @@ size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
         f.normed = fptr(d, norm->out);
         f.eps = norm->plan.eps;
     }
-    // the norm inside the GEMV's prologue, or ahead of the launch on its own
-    const auto run = [&]() -> hipError_t {
-        if (norm && !gemv_dense_norm_takes(f)) {
-            const hipError_t e = launch_rms_norm(f.a, f.gamma, f.normed, f.m, f.k, f.eps, d->stream);
-            if (e != hipSuccess) return e;
+    // The norm runs inside the GEMV's prologue, or ahead of the launch on its
+    // own; the products then read its output, whose alignment counts and not
+    // the input's. Settled here, before anything is launched: false where no
+    // kernel takes what the launch would be given.
+    const auto settle = [&]() -> bool {
+        if (norm && !(gemv_dense_takes(f) && gemv_dense_norm_takes(f))) {
             f.a = f.normed;
             f.gamma = nullptr;
+        }
+        return gemv_dense_takes(f) || gemm_dense_takes(f);
+    };
+    const auto run = [&]() -> hipError_t {
+        if (norm && f.gamma == nullptr) {
+            const hipError_t e = launch_rms_norm(fptr(d, norm->in[0]), fptr(d, norm->in[1]), f.normed, f.m, f.k, f.eps,
+                                                 d->stream);
+            if (e != hipSuccess) return e;
         }
         const hipError_t e = launch_gemv_dense(f, d->stream);
         return e == hipErrorNotSupported ? launch_gemm_dense(f, Workspace{d->workspace, d->workspace_floats}, d->stream)
@@ -848,10 +857,7 @@ size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
                 ++used;
             }
         }
-        GemvDense plain = f;  // as the GEMM would be given it
-        plain.gamma = nullptr;
-        if (norm) plain.a = f.normed;
-        if (used == 1 || !(gemv_dense_takes(f) || gemm_dense_takes(plain))) return 0;
+        if (used == 1 || !settle()) return 0;
         *err = run();
         d->stats.fused_commands += used;
         return used;
@@ -883,7 +889,7 @@ size_t try_fuse_dense(Device* d, size_t i, hipError_t* err) {
         g.m = rows;
         g.k = inter;
         g.epilogue = kFusedPlain;
-        if (!gemv_dense_takes(f) || !gemv_dense_takes(g)) return 0;
+        if (!settle() || !gemv_dense_takes(g)) return 0;
         size_t used = (j - i) + 1;
         if (j + 1 < n) {
             const Logged& add = d->log[j + 1];

@@ -139,6 +139,57 @@ def test_dense_decode_units_fuse(hip, rows, hidden, inter):
     assert_normwise(hip.read_f32(buf["f"].buffer, buf["f"].len), f)
 
 
+# Every operand of the units off 16-byte alignment in turn (index: floats to
+# start at), in the forms with the norm inside the launch, ahead of it, and ahead
+# of the GEMM: commands no dense kernel takes as a unit run one by one.
+@pytest.mark.parametrize("off", ["x", "gamma", "normed", "w", "gate", "down", "resid", "out"])
+@pytest.mark.parametrize("rows,hidden", [(1, 256), (4, 256), (2, 260), (5, 256), (32, 256), (40, 256)])
+def test_units_with_an_unaligned_operand(hip, rows, hidden, off):
+    r = np.random.default_rng(rows + hidden)
+    inter, n = 48, 36
+
+    def put(name, *shape):
+        x = r.uniform(-1, 1, shape).astype(np.float32)
+        at = 1 if name == off else 0
+        return x, BufferRef(hip.upload_new_f32(np.concatenate([np.zeros(at, np.float32), x.ravel()])), at, x.size)
+
+    def room(name, width):
+        at = 1 if name == off else 0
+        return BufferRef(hip.allocate_f32(rows * width + at, 256), at, rows * width)
+
+    x, xr = put("x", rows, hidden)
+    g, gr = put("gamma", hidden)
+    (w, wr), (w2, w2r) = put("w", n, hidden), put("", n, hidden)
+    (gate, gater), (up, upr), (down, downr) = put("gate", inter, hidden), put("", inter, hidden), put("down", hidden, inter)
+    res, resr = put("resid", rows, n)
+    res2, res2r = put("resid", rows, hidden)
+    normed, one, two, added = room("normed", hidden), room("out", n), room("", n), room("out", n)
+    normed2, f, added2 = room("normed", hidden), room("out", hidden), room("out", hidden)
+    f32 = Value.f32
+    act, gv, on, wv = f32([rows, hidden]), f32([hidden], ValueRole.PARAM), f32([rows, n]), f32([n, hidden])
+    hip.dispatch(Op.rms_norm(1e-5), [xr, gr], [act, gv], [normed], [act])
+    hip.dispatch(Op.matmul_nt(), [normed, wr], [act, wv], [one], [on])
+    hip.dispatch(Op.matmul_nt(), [normed, w2r], [act, wv], [two], [on])
+    hip.dispatch(Op.add(), [resr, two], [on, on], [added], [on])
+    hip.dispatch(Op.rms_norm(1e-5), [xr, gr], [act, gv], [normed2], [act])
+    hip.dispatch(Op.swiglu(), [normed2, gater, upr, downr],
+                 [act, f32([inter, hidden]), f32([inter, hidden]), f32([hidden, inter])], [f], [act])
+    hip.dispatch(Op.add(), [res2r, f], [act, act], [added2], [act])
+    hip.synchronize()
+
+    def got(ref):
+        return hip.read_f32(ref.buffer, ref.offset + ref.len)[ref.offset:]
+
+    want = oracle.rms_norm(x.ravel(), g, rows, hidden, 1e-5)
+    for ref in (normed, normed2):
+        assert_normwise(got(ref), want)
+    assert_normwise(got(one), oracle.matmul_nt(want, w.ravel(), 1, rows, hidden, n))
+    assert_normwise(got(two), oracle.matmul_nt(want, w2.ravel(), 1, rows, hidden, n))
+    assert np.array_equal(got(added), res.ravel() + got(two))
+    assert_normwise(got(f), oracle.swiglu(want, gate.ravel(), up.ravel(), down.ravel(), rows, hidden, inter))
+    assert np.array_equal(got(added2), res2.ravel() + got(f))
+
+
 def test_units_with_overlapping_regions_keep_the_command_order(hip):
     """A projection that writes over another's weight, or reads a weight the
     norm before it wrote, gives what the commands give one after the other."""
