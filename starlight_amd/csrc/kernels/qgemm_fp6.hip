@@ -213,7 +213,9 @@ __global__ __launch_bounds__(256) void split_fp6(const float* __restrict__ a, co
         uint32_t m = max(max(mag4(v[0]), mag4(v[1])), max(mag4(v[2]), mag4(v[3])));
         m = max(m, static_cast<uint32_t>(dpp_i<kDppXor1>(static_cast<int>(m))));
         if (w >= units) return;
-        const int e = mag_exp(m);
+        // (a block of zeros takes the row's exponent: 0 would lie 127 and more
+        // above that of a row of denormals, where the scale's byte is NaN's)
+        const int e = m != 0 ? mag_exp(m) : er;
         const bool finite = m < 0x7f800000u;
         const uint32_t b = w / 2 % 4;
         uint8_t* const dst = rec + static_cast<uint64_t>(w / 8) * kRecord;

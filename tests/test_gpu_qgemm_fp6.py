@@ -90,6 +90,21 @@ def test_extreme_magnitudes(hip, scale):
     assert np.all(err <= 1e-5 * np.sqrt(256) * 8 * 0.05 * scale + 2e-45)
 
 
+# (2^-129 and 2^-128: the smallest and largest maximum with exponent -128)
+@pytest.mark.parametrize("top", [2.0**-149, 2.0**-141, 2.0**-129, 1.5 * 2.0**-129, 2.0**-128, 2.0**-126])
+def test_zero_blocks_in_a_row_of_denormals(hip, top):
+    r = np.random.default_rng(10)
+    a = (r.uniform(-1, 1, (20, 384)) * top).astype(np.float32)
+    a[:, 5] = top
+    a[:, 32:64] = 0.0
+    a[:, 128:256] = 0.0
+    w = weight(hip, 40, 384, 128, r)
+    got = run(hip, a, w)
+    want = a.astype(np.float64) @ w[2].T
+    # (sums of 224 products of at most 0.4 top, and a result's own rounding)
+    assert np.all(np.abs(got - want) <= 224 * 0.4 * top * 2.0**-22 + 2.0**-149)
+
+
 def test_infinities_and_nan_stay_in_their_row(hip):
     r = np.random.default_rng(6)
     a = r.standard_normal((40, 384)).astype(np.float32)
