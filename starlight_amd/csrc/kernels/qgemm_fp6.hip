@@ -217,6 +217,7 @@ __global__ __launch_bounds__(256) void split_fp6(const float* __restrict__ a, co
         // above that of a row of denormals, where the scale's byte is NaN's)
         const int e = m != 0 ? mag_exp(m) : er;
         const bool finite = m < 0x7f800000u;
+        const bool held = finite && kOne + e - er >= 0;  // else below what a block scale can say: zero digits
         const uint32_t b = w / 2 % 4;
         uint8_t* const dst = rec + static_cast<uint64_t>(w / 8) * kRecord;
         constexpr int kBias = 16 * (1 + 32 + 1024 + 32768 + 1048576);  // makes every digit d + 16 >= 0
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256) void split_fp6(const float* __restrict__ a, co
         for (int q = 0; q < 4; ++q) {
             const float f[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) x[4 * q + i] = finite ? __float2int_rn(ldexpf(f[i], 24 - e)) + kBias : kBias;
+            for (int i = 0; i < 4; ++i) x[4 * q + i] = held ? __float2int_rn(ldexpf(f[i], 24 - e)) + kBias : kBias;
         }
 #pragma unroll
         for (int j = 0; j < kDigits; ++j) {

@@ -105,6 +105,21 @@ def test_zero_blocks_in_a_row_of_denormals(hip, top):
     assert np.all(np.abs(got - want) <= 224 * 0.4 * top * 2.0**-22 + 2.0**-149)
 
 
+# a block below 2^-127 of its row's maximum (the first one's, under zero codes)
+# may be dropped, but not raised to that
+@pytest.mark.parametrize("top,rest", [(1e30, 1e-30), (3e38, 2.0**-3), (1.0, 2.0**-140), (2.0**120, 2.0**-8)])
+def test_blocks_below_the_range_of_a_block_scale(hip, top, rest):
+    r = np.random.default_rng(12)
+    a = (r.uniform(0.5, 1, (20, 256)) * rest).astype(np.float32)
+    a[:, :32] = top
+    codes = r.integers(1, 8, (24, 256)).astype(np.int8)
+    codes[:, :32] = 0
+    w = weight(hip, 24, 256, 128, r, codes)
+    got = run(hip, a, w)
+    want = a.astype(np.float64) @ w[2].T
+    assert np.all(got >= 0) and np.all(got <= want * (1 + 2.0**-20) + 2.0**-148)
+
+
 def test_infinities_and_nan_stay_in_their_row(hip):
     r = np.random.default_rng(6)
     a = r.standard_normal((40, 384)).astype(np.float32)
