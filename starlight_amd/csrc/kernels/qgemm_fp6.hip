@@ -6,34 +6,46 @@
 // holds every integer of magnitude at most 16 exactly (as n / 8, with the
 // sign-magnitude code n itself), so an INT4 code is one E2M3 value. Of every
 // activation row, each 32 elements that one lane feeds to a product share an
-// exponent E (|a| < 2^E) and become integers X = rint(a * 2^(24 - E)), cut
-// into five signed base-32 digits, X = sum_j d_j 32^j with |d_j| <= 16, each
-// one E2M3 value as well: 24 significant bits below the block's largest
-// element. The products d_j * q are exact, and the instruction's block scales
-// carry 2^E (relative to the row's largest exponent) and 32^j. A product's sum
-// over its 128 k is exact where the blocks' exponents are close, but adding
-// it to a larger sum rounds down by up to 2^-23 of that: chained over all five
-// digits, the errors of a whole model's logits grew 1.2 to 2.4 times. So the
-// three low digits and the two high ones are summed apart (the high sum needs
-// 19 bits plus the exponents' spread), added in f32, multiplied by the
-// group's scale, added to the f32 result, and that is scaled back by the
-// row's exponent at the end. Error against float64 as the fp16 split's
-// (qgemm_mfma.hip) or below: [4096 x 14336] at M = 1024 1.5e-7 against 1.7e-7,
-// [28672 x 4096] 1.3e-7 against 1.4e-7; whole models the same.
+// exponent E (|a| < 2^E) and become integers X = rint(a * 2^(29 - E)), cut
+// into six signed base-32 digits, X = sum_j d_j 32^j with |d_j| <= 16, each
+// one E2M3 value as well: 29 bits below 2^E. A block most of whose elements
+// (17 or more nonzero ones) lie below 2^(E - 8), under an outlier channel for
+// instance, gets two more digits, 39 bits. So an element keeps at least the 22
+// bits it has as two fp16 parts (qgemm_mfma.hip), or the block's small ones do
+// statistically: with five digits a channel at 1,000 times the others, in each
+// 32 and under zero codes, left those an error of 2e-5. The products d_j * q
+// are exact, and the instruction's block scales carry 2^E (relative to the
+// row's largest exponent) and 32^j. A product's sum over its 128 k is exact
+// where the blocks' exponents are close, but adding it to a larger sum cuts
+// that downwards by up to 2^-23 of it: chained over all digits, the errors of
+// a whole model's logits grew 1.2 to 2.4 times. So the four low digits and the
+// two high ones are summed apart (the high sum needs 20 bits plus the
+// exponents' spread), added in f32, multiplied by the group's scale, added to
+// the f32 result, and that is scaled back by the row's exponent at the end.
+//
+// Error against float64, normwise, fp16 split / this: activations normal, silu
+// of a normal times another, Student t with 3 and 2 degrees, cubed Laplace, one
+// channel or one in each 32 at 30 to 100,000 times the others with and without
+// codes under it: k = 512 1.1e-7 to 1.8e-7 / 4.6e-8 to 7.6e-8, k = 4096 1.3e-7
+// to 2.7e-7 / 7.3e-8 to 9.6e-8, k = 14336 1.7e-7 to 3.2e-7 / 9.0e-8 to 1.2e-7.
 //
 // Rate. Register-resident loops on MI355X reach 8.43 PFLOP/s with 6-bit
-// operands and 2.17 PFLOP/s with fp16 ones: five 6-bit products per multiply
-// allow 1.69 PFLOP/s of f32 result, two fp16 ones 1.08. With the split, against
-// the fp16 route: [28672 x 4096] M = 1024 358 us against 525 (673 TFLOP/s of
-// f32 result), M = 77 58 against 89; [4096 x 14336] M = 1024 212 against 304,
-// M = 512 117 against 186, M = 77 41 against 159; [4096 x 4096] M = 77 24
-// against 56. What bounds it now: vector and matrix instructions of a SIMD's
-// waves do not overlap here, and a 64 x 256 tile's pass has 80 products (1,280
-// cycles) and about 160 vector instructions (640) per wave, two waves per
-// SIMD: 3,840 of about 6,000 cycles measured; LDS is busy a third of the time.
-// Deeper operand prefetch and wave priorities changed nothing, and gathering
-// the records in operand order from memory (no LDS conflicts, scattered
-// 64-byte loads) was slower.
+// operands and 2.17 PFLOP/s with fp16 ones: six 6-bit products per multiply
+// allow 1.41 PFLOP/s of f32 result, two fp16 ones 1.08. With the split, against
+// the fp16 route (and five digits): [28672 x 4096] M = 1024 398 us against 525
+// (355; 604 TFLOP/s of f32 result), M = 77 65 against 89 (58); [4096 x 14336] M =
+// 1024 238 against 304 (213), M = 512 130 against 186 (117), M = 77 46 against
+// 159 (41); [4096 x 4096] M = 77 26 against 56 (25). What bounds it now: vector
+// and matrix instructions of a SIMD's waves do not overlap here, and a 64 x 256
+// tile's pass has 96 products (1,536 cycles) and about 170 vector instructions
+// (680) per wave, two waves per SIMD: 4,430 of about 6,500 cycles measured; LDS
+// is busy for 2,950 of them (reads of the digits, and the stage's writes in the
+// middle of the pass: at its end, 1-2% slower; loads straight into LDS the same
+// time as through registers). Deeper operand prefetch and wave priorities
+// changed nothing, and gathering the records in operand order from memory (no
+// LDS conflicts, scattered 64-byte loads) was slower. A sixth digit only for
+// blocks that need it costs as much where they are few (the LDS room and the
+// branch) and more behind silu(g) * u, where nearly every tile has one.
 //
 // Kernels
 //  * repack_fp6 (bind): the codes as E2M3 in operand order, per 16-row tile
@@ -42,12 +54,13 @@
 //    i < 32, of the superblock (the order in which a quad of threads reads
 //    whole float4 of the activations);
 //  * split_fp6: one block per row: row maximum, block exponents, digits. A
-//    record of 512 bytes per row and superblock: five digit planes of 4 lanes
-//    x 16 then 4 x 8 bytes, and the four block scales;
-//  * qgemm_fp6: records staged through LDS in rows of 528 bytes (the 16 rows
-//    of one operand read fall on disjoint groups of 4 banks), shared by the
-//    block's waves; weights straight from memory into registers, one
-//    superblock ahead.
+//    record of 592 bytes per superblock and row: six digit planes of 4 lanes
+//    x 16 then 4 x 8 bytes, and four block scales with the flag of further
+//    digits, which lie in planes of their own;
+//  * qgemm_fp6: a block's rows of a superblock, contiguous, staged through LDS
+//    as they are (592 bytes a row: the 16 rows of one operand read fall on
+//    disjoint groups of 4 banks), shared by the block's waves; weights straight
+//    from memory into registers, one superblock ahead.
 #include "common.h"
 #include "kernels.h"
 #include "qgemm_act.h"
@@ -60,17 +73,31 @@ namespace {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int kDigits = 5, kLowDigits = 3;
-constexpr uint32_t kRecord = 512;     // bytes per row and superblock
-constexpr uint32_t kPlane = 96;       // bytes of one digit of a record
-constexpr uint32_t kScalesAt = kDigits * kPlane;
-constexpr uint32_t kLdsRow = kRecord + 16;
+constexpr int kDigits = 6, kLowDigits = 4;    // digits of every element, and of the low sum
+constexpr int kMoreDigits = 2;                // of a block whose maximum stands far above most of it
+constexpr int kFar = 8;                       // powers of two that is
+constexpr uint32_t kPlane = 96;               // bytes of one digit of a row and superblock
+constexpr uint32_t kScalesAt = kDigits * kPlane;  // 16 bits per lane: block scale, kFurther
+constexpr int kFurther = 256;
+constexpr uint32_t kRecord = 592;                 // bytes per row and superblock, also of its row in LDS
+constexpr uint32_t kMore = kMoreDigits * kPlane;  // bytes of the further digits of a row and superblock
+static_assert(kScalesAt + 8 <= kRecord && kRecord % 16 == 0, "record layout");
 constexpr uint32_t kTileBytes = 1536;           // one 16-row weight tile of one superblock
+constexpr uint32_t kPad = 128 * kRecord + 8192;  // bytes a block's loads may reach past the last record
 constexpr int kOne = 127;                       // E8M0 of 1.0
 
 // Sign and magnitude of d, |d| <= 16: the E2M3 code of d / 8.
 __device__ __forceinline__ uint32_t e2m3(int d) {
     return static_cast<uint32_t>(max(d, -d)) | (static_cast<uint32_t>(d >> 26) & 32u);
+}
+
+// The same of digit j of x, a sum of 32^j (d_j + 16) with every d_j + 16 < 32
+// but the highest's (4 instructions, not 7: digits are most of the split's).
+__device__ __forceinline__ uint32_t digit(int x, int j, bool highest) {
+    const uint32_t u = static_cast<uint32_t>(x);
+    if (highest) return e2m3(static_cast<int>(u >> (5 * j)) - 16);
+    const uint32_t sign = j == 0 ? ~u << 1 : ~u >> (5 * j - 1);
+    return __builtin_amdgcn_sad_u8(u >> (5 * j) & 31u, 16u, 0u) | (sign & 32u);
 }
 
 // Element i of lane l within a superblock.
@@ -133,10 +160,12 @@ __device__ __forceinline__ int mag_exp(uint32_t mag) {
 // u is half h = u % 2 (elements 16 h ..) of lane block b = u / 2 % 4 of
 // superblock u / 8. With gamma (NP <= 2), of RMSNorm(a) * gamma; NP == 0 reads
 // the row twice instead of holding it. Bound by the vector unit's work on the
-// digits and by its reads; M = 1024, k = 4096: see qgemm_fp6.
+// digits and by its reads; M = 1024: k = 4096 12.3 us, silu(a) * u at k = 14336
+// 53 (174 MB read and written, 3.3 TB/s, with two waves per SIMD).
 template <int NP>
 __global__ __launch_bounds__(256) void split_fp6(const float* __restrict__ a, const float* __restrict__ u,
-                                                 uint8_t* __restrict__ records, int* __restrict__ row_exp, uint32_t k,
+                                                 uint8_t* __restrict__ records, uint8_t* __restrict__ more,
+                                                 int* __restrict__ row_exp, uint32_t k,
                                                  const float* __restrict__ gamma, float eps) {
     __shared__ float scratch[4];
     __shared__ uint32_t scratch_u[4];
@@ -207,49 +236,78 @@ __global__ __launch_bounds__(256) void split_fp6(const float* __restrict__ a, co
     }
     const int er = mag_exp(block_max_u32(mx, scratch_u));
     if (threadIdx.x == 0) row_exp[r] = er;
-    uint8_t* const rec = records + r * (k / 128) * kRecord;
+    const uint64_t m = gridDim.x;
+    // One plane of 16 elements' codes: half h of lane block b.
+    const auto store = [](uint8_t* plane, uint32_t h, uint32_t b, const uint32_t (&c)[16]) {
+        const uint32_t w0 = c[0] | c[1] << 6 | c[2] << 12 | c[3] << 18 | c[4] << 24 | c[5] << 30;
+        const uint32_t w1 = c[5] >> 2 | c[6] << 4 | c[7] << 10 | c[8] << 16 | c[9] << 22 | c[10] << 28;
+        const uint32_t w2 = c[10] >> 4 | c[11] << 2 | c[12] << 8 | c[13] << 14 | c[14] << 20 | c[15] << 26;
+        uint32_t* const hi = reinterpret_cast<uint32_t*>(plane) + 4 * b;
+        if (h == 0) {
+            hi[0] = w0;
+            hi[1] = w1;
+            hi[2] = w2;
+        } else {
+            hi[3] = w0;
+            *reinterpret_cast<uint2*>(plane + 64 + 8 * b) = make_uint2(w1, w2);
+        }
+    };
     // Unit w's digits; its lane block's other half is in the neighbouring thread.
     auto put = [&](uint32_t w, const float4 (&v)[4]) {
-        uint32_t m = max(max(mag4(v[0]), mag4(v[1])), max(mag4(v[2]), mag4(v[3])));
-        m = max(m, static_cast<uint32_t>(dpp_i<kDppXor1>(static_cast<int>(m))));
-        if (w >= units) return;
+        uint32_t mx32 = max(max(mag4(v[0]), mag4(v[1])), max(mag4(v[2]), mag4(v[3])));
+        mx32 = max(mx32, static_cast<uint32_t>(dpp_i<kDppXor1>(static_cast<int>(mx32))));
         // (a block of zeros takes the row's exponent: 0 would lie 127 and more
         // above that of a row of denormals, where the scale's byte is NaN's)
-        const int e = m != 0 ? mag_exp(m) : er;
-        const bool finite = m < 0x7f800000u;
+        const int e = mx32 != 0 ? mag_exp(mx32) : er;
+        const bool finite = mx32 < 0x7f800000u;
+        float f[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) f[4 * q] = v[q].x, f[4 * q + 1] = v[q].y, f[4 * q + 2] = v[q].z, f[4 * q + 3] = v[q].w;
+        // (of its 32 elements, 17 or more nonzero and below 2^(e - kFar))
+        const uint32_t least = max(__float_as_uint(ldexpf(1.0f, e - kFar)), 1u) - 1u;
+        int small = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) small += (__float_as_uint(f[i]) & 0x7fffffffu) - 1u < least ? 1 : 0;
+        small += dpp_i<kDppXor1>(small);
+        if (w >= units) return;
         const bool held = finite && kOne + e - er >= 0;  // else below what a block scale can say: zero digits
-        const uint32_t b = w / 2 % 4;
-        uint8_t* const dst = rec + static_cast<uint64_t>(w / 8) * kRecord;
-        constexpr int kBias = 16 * (1 + 32 + 1024 + 32768 + 1048576);  // makes every digit d + 16 >= 0
+        const bool further = held && small > 16;
+        const uint32_t h = w % 2, b = w / 2 % 4;
+        const uint64_t at = w / 8 * m + r;
+        uint8_t* const dst = records + at * kRecord;
+        constexpr int kBias = 16 * (1 + 32 + 1024 + 32768 + 1048576 + 33554432);  // makes every digit d + 16 >= 0
         int x[16];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float f[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[4 * q + i] = held ? __float2int_rn(ldexpf(f[i], 24 - e)) + kBias : kBias;
-        }
+        for (int i = 0; i < 16; ++i) x[i] = held ? __float2int_rn(ldexpf(f[i], 29 - e)) + kBias : kBias;
 #pragma unroll
         for (int j = 0; j < kDigits; ++j) {
             uint32_t c[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) c[i] = e2m3((j == kDigits - 1 ? x[i] >> 20 : (x[i] >> (5 * j)) & 31) - 16);
-            const uint32_t w0 = c[0] | c[1] << 6 | c[2] << 12 | c[3] << 18 | c[4] << 24 | c[5] << 30;
-            const uint32_t w1 = c[5] >> 2 | c[6] << 4 | c[7] << 10 | c[8] << 16 | c[9] << 22 | c[10] << 28;
-            const uint32_t w2 = c[10] >> 4 | c[11] << 2 | c[12] << 8 | c[13] << 14 | c[14] << 20 | c[15] << 26;
-            uint32_t* const hi = reinterpret_cast<uint32_t*>(dst + j * kPlane) + 4 * b;
-            if (w % 2 == 0) {
-                hi[0] = w0;
-                hi[1] = w1;
-                hi[2] = w2;
-            } else {
-                hi[3] = w0;
-                *reinterpret_cast<uint2*>(dst + j * kPlane + 64 + 8 * b) = make_uint2(w1, w2);
-            }
+            for (int i = 0; i < 16; ++i) c[i] = digit(x[i], j, j == kDigits - 1);
+            store(dst + j * kPlane, h, b, c);
         }
         // the block's power of two against the row's; 255 (NaN) where the
         // block holds an infinity or NaN: its row's results are NaN then, as
         // infinity minus its own high part is in an fp16 split
-        if (w % 2 == 0) dst[kScalesAt + b] = finite ? static_cast<uint8_t>(max(kOne + e - er, 0)) : 255u;
+        if (h == 0)
+            reinterpret_cast<uint16_t*>(dst + kScalesAt)[b] =
+                static_cast<uint16_t>((finite ? max(kOne + e - er, 0) : 255) | (further ? kFurther : 0));
+        if (further) {
+            // what the digits leave, at most half a unit (exact: a value
+            // of 2^24 units or more is whole), in 1024ths of it: |.| <= 512
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float t = ldexpf(f[i], 29 - e);
+                x[i] = __float2int_rn((t - rintf(t)) * 1024.0f) + 16 * (1 + 32);
+            }
+#pragma unroll
+            for (int j = 0; j < kMoreDigits; ++j) {
+                uint32_t c[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) c[i] = e2m3((j == kMoreDigits - 1 ? x[i] >> 5 : x[i] & 31) - 16);
+                store(more + at * kMore + j * kPlane, h, b, c);
+            }
+        }
     };
     if constexpr (NP > 0) {
 #pragma unroll
@@ -275,7 +333,8 @@ struct Fp6Seg {
 };
 
 struct Fp6Args {
-    const uint8_t* records;
+    const uint8_t* records;  // [superblock][row]
+    const uint8_t* more;     // the same, written where a block has further digits
     const int* row_exp;
     Fp6Seg seg[kFusedMaxSegs];
     uint32_t nseg, m, sb_total, rows, cols;  // rows, cols: row and column blocks
@@ -299,13 +358,15 @@ __device__ __forceinline__ T load_at(__attribute__((address_space(1))) const uin
 // digit sums in accumulation registers and moves each out before the vector
 // unit can add it, 128 moves in a 64 x 256 tile's pass (396 -> 360 us).
 template <int MT, int NT, int WM, int WN>
-__global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2))) void qgemm_fp6(Fp6Args p) {
+__global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(MT * NT <= 4 ? 4 : 2))) void qgemm_fp6(Fp6Args p) {
     constexpr int T = kWave * WM * WN;
     constexpr uint32_t BM = 16 * MT * WM, BN = 16 * NT * WN;
-    constexpr int NL = BM * 32 / T;  // 16-byte pieces of a stage per thread
-    static_assert(NL * T == BM * 32, "whole pieces per thread");
+    // 16-byte pieces of a stage per thread, the last ones past its BM rows (kPad)
+    constexpr int NL = (BM * (kRecord / 16) + T - 1) / T;
+    static_assert(NL * T * 16 <= kPad, "a whole stage past the last record");
     prefetch_kernarg<arg_bytes<Fp6Args>()>();
-    __shared__ __align__(16) uint8_t as[2][BM * kLdsRow];
+    constexpr uint32_t kBuf = NL * T * 16;
+    __shared__ __align__(16) uint8_t as[2 * kBuf];
     const uint32_t tid = threadIdx.x, lane = tid % kWave;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave), wm = wave / WN, wn = wave % WN;
     // Blocks go to the 8 XCDs round robin; each XCD takes a contiguous run of
@@ -331,10 +392,6 @@ __global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2
         uint2 hi[NT];
         float s[NT];
     };
-    uint32_t src[NL];  // byte offsets of this thread's pieces: piece tid % 32 of rows tid / 32 + T / 32 i
-#pragma unroll
-    for (int i = 0; i < NL; ++i)
-        src[i] = (min(m0 + tid / 32 + T / 32 * i, p.m - 1) * p.sb_total * (kRecord / 16) + tid % 32) * 16;
     // A uniform base that stays in scalar registers plus a 32-bit lane offset
     // per load: left to itself the compiler keeps one 64-bit vector address
     // per load.
@@ -352,12 +409,13 @@ __global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2
         wt[j] = SL_GSEG(tiles) + t * kTileBytes;
         ws[j] = SL_GSEG(scales) + t * 16;
     }
-    const uint32_t lane16 = lane * 16, lane8 = lane * 8, col4 = lane % 16 * 4;
+    const uint32_t tid16 = tid * 16, lane16 = lane * 16, lane8 = lane * 8, col4 = lane % 16 * 4;
     auto load_stage = [&](uint32_t sb) -> Stage {
         Stage r;
-        global_u8* const base = scalar(p.records + static_cast<uint64_t>(sb) * kRecord);
+        // (rows past m are the next superblock's, or kPad: computed, not stored)
+        const uint8_t* const rec = p.records + (static_cast<uint64_t>(sb) * p.m + m0) * kRecord;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) r.v[i] = load_at<uint4>(base + src[i]);
+        for (int i = 0; i < NL; ++i) r.v[i] = load_at<uint4>(scalar(rec + T * 16 * i) + tid16);
         return r;
     };
     auto load_weights = [&](uint32_t sb) -> Weights {
@@ -375,21 +433,24 @@ __global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2
         uint4 lo;
         uint2 hi;
     };
-    auto row_of = [&](uint32_t buf, int i) -> const uint8_t* {
-        return &as[buf][(16 * (wm * MT + i) + lane % 16) * kLdsRow];
+    const auto operand = [](const Digit x) -> v8i {
+        return v8i{static_cast<int>(x.lo.x), static_cast<int>(x.lo.y), static_cast<int>(x.lo.z),
+                   static_cast<int>(x.lo.w), static_cast<int>(x.hi.x), static_cast<int>(x.hi.y), 0, 0};
     };
-    auto read_digit = [&](uint32_t buf, int q) -> Digit {  // digit q % kDigits of row tile q / kDigits
-        const uint8_t* const at = row_of(buf, q / kDigits) + q % kDigits * kPlane;
-        return Digit{*reinterpret_cast<const uint4*>(at + 16 * (lane / 16)),
-                     *reinterpret_cast<const uint2*>(at + 64 + 8 * (lane / 16))};
+    // LDS addresses: one register per use that the pass's buffer is added to,
+    // the rest as the instructions' 16-bit offsets (both buffers' addresses as
+    // constants do not fit those and took 34 registers more than there are)
+    const auto opaque = [](uint32_t v) -> uint32_t {
+        asm volatile("" : "+v"(v));
+        return v;
     };
-    auto read_scale = [&](uint32_t buf, int i) -> int { return row_of(buf, i)[kScalesAt + lane / 16]; };
+    const uint32_t row0 = (16 * wm * MT + lane % 16) * kRecord;
+    auto read_plane = [&](uint32_t at16, uint32_t at8, int i, int plane) -> Digit {  // of row tile i
+        const uint32_t o = i * 16 * kRecord + plane * kPlane;
+        return Digit{*reinterpret_cast<const uint4*>(as + at16 + o), *reinterpret_cast<const uint2*>(as + at8 + o)};
+    };
     constexpr int kArithmetic = 0xF, kAhead = 1;
-    auto store_stage = [&](uint32_t buf, const Stage r) {
-#pragma unroll
-        for (int i = 0; i < NL; ++i)
-            *reinterpret_cast<uint4*>(&as[buf][(tid / 32 + T / 32 * i) * kLdsRow + tid % 32 * 16]) = r.v[i];
-    };
+    auto store_piece = [&](uint32_t at, const Stage& r, int i) { *reinterpret_cast<uint4*>(as + at + T * 16 * i) = r.v[i]; };
 
     v4f acc[MT][NT];
 #pragma unroll
@@ -409,41 +470,90 @@ __global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2
         __builtin_amdgcn_sched_barrier(kArithmetic);
         Digit ring[kAhead + 1];
         int scale[MT];
+        const uint32_t row = row0 + buf * kBuf, at16 = opaque(row + 16 * (lane / 16)),
+                       at8 = opaque(row + 64 + 8 * (lane / 16)), at2 = row + kScalesAt + 2 * (lane / 16);
 #pragma unroll
-        for (int i = 0; i < MT; ++i) scale[i] = read_scale(buf, i);
+        for (int i = 0; i < MT; ++i) scale[i] = *reinterpret_cast<const uint16_t*>(as + at2 + i * 16 * kRecord);
 #pragma unroll
-        for (int q = 0; q < kAhead; ++q) ring[q] = read_digit(buf, q);
+        for (int q = 0; q < kAhead; ++q) ring[q] = read_plane(at16, at8, q / kDigits, q % kDigits);
+        const auto product = [&](const Digit x, int j, const v4f c, int scale_a, int e) -> v4f {
+            return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(operand(x), operand(Digit{w.lo[j], w.hi[j]}), c, 2, 2,
+                                                                    0, scale_a, 0, kOne + e);
+        };
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        // With further digits anywhere, the whole pass is left to its end (below)
+        // and adds nothing here.
+        int flags = scale[0];
+#pragma unroll
+        for (int i = 1; i < MT; ++i) flags |= scale[i];
+        const bool wide = __builtin_amdgcn_ballot_w64(flags >= kFurther) != 0;  // wave-uniform
+        float here[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) here[j] = wide ? 0.f : w.s[j];
+        const uint32_t to = opaque(tid16 + (buf ^ 1) * kBuf);
         v4f lo[NT], hi[NT];
 #pragma unroll
         for (int q = 0; q < MT * kDigits; ++q) {
-            if (q + kAhead < MT * kDigits) ring[(q + kAhead) % (kAhead + 1)] = read_digit(buf, q + kAhead);
+            // the next stage's pieces, in the middle of the pass
+            if (const int a = q - (MT * kDigits - NL) / 2; a >= 0 && a < NL) store_piece(to, st, a);
+            if (const int a = q + kAhead; a < MT * kDigits)
+                ring[a % (kAhead + 1)] = read_plane(at16, at8, a / kDigits, a % kDigits);
             __builtin_amdgcn_sched_barrier(kArithmetic);
             const int i = q / kDigits, d = q % kDigits;
             const Digit x = ring[q % (kAhead + 1)];
-            const v8i av = {static_cast<int>(x.lo.x), static_cast<int>(x.lo.y), static_cast<int>(x.lo.z),
-                            static_cast<int>(x.lo.w), static_cast<int>(x.hi.x), static_cast<int>(x.hi.y), 0, 0};
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                const v8i bv = {static_cast<int>(w.lo[j].x), static_cast<int>(w.lo[j].y),
-                                static_cast<int>(w.lo[j].z), static_cast<int>(w.lo[j].w),
-                                static_cast<int>(w.hi[j].x), static_cast<int>(w.hi[j].y), 0, 0};
                 v4f& t = d < kLowDigits ? lo[j] : hi[j];
-                const v4f c = d == 0 || d == kLowDigits ? v4f{0.f, 0.f, 0.f, 0.f} : t;
-                t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 2, 2, 0, scale[i], 0,
-                                                                     kOne + 5 * (d - (kDigits - 1)));
+                t = product(x, j, d == 0 || d == kLowDigits ? zero : t, scale[i], 5 * (d - (kDigits - 1)));
             }
             if (d == kDigits - 1)
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(hi[j][e] + lo[j][e], w.s[j], acc[i][j][e]);
+                    for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(hi[j][e] + lo[j][e], here[j], acc[i][j][e]);
         }
-        store_stage(buf ^ 1, st);
+        // Further digits: elements of a block 2^8 and more apart. The sum of a plane is still exact or close, the four low planes' together is not, and
+        // is cut always downwards (a bias of 5e-7 over 129 superblocks), so each
+        // plane starts from zero here and f32 additions, which round to nearest,
+        // join them from the lowest on. (A row past m may show another row's
+        // flag: it reads row m - 1's further digits and stores nothing.)
+        if (wide) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                v4f sum[NT];
+#pragma unroll
+                for (int j = 0; j < NT; ++j) sum[j] = zero;
+#pragma unroll 1
+                for (int d = -kMoreDigits; d < kDigits; ++d) {
+                    Digit x{make_uint4(0u, 0u, 0u, 0u), make_uint2(0u, 0u)};
+                    if (d >= 0) {
+                        x = read_plane(at16, at8, i, d);
+                    } else if (scale[i] >= kFurther) {
+                        const uint32_t l = opaque(lane);  // addresses made here, not kept over the loop
+                        const uint32_t r = min(m0 + 16 * (wm * MT + i) + l % 16, p.m - 1);
+                        const uint8_t* const at = p.more + (static_cast<uint64_t>(sb) * p.m + r) * kMore +
+                                                  (d + kMoreDigits) * kPlane + 8 * (l / 16);
+                        x = Digit{*reinterpret_cast<const uint4*>(at + 8 * (l / 16)),
+                                  *reinterpret_cast<const uint2*>(at + 64)};
+                    }
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) sum[j] += product(x, j, zero, scale[i], 5 * (d - (kDigits - 1)));
+                }
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(sum[j][e], w.s[j], acc[i][j][e]);
+            }
+        }
         __syncthreads();
         return wx;
     };
     Weights w0 = load_weights(beg);
-    store_stage(0, load_stage(beg));
+    {
+        const Stage st = load_stage(beg);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) store_piece(tid16, st, i);
+    }
     __syncthreads();
     // two passes per iteration: the weights' registers alternate, not moved
     uint32_t sb = beg;
@@ -484,12 +594,15 @@ __global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(2
         }
 }
 
+// Records, then what a last block's loads read past them, the further
+// digits, and the row exponents, in the workspace.
 struct RecordLayout {
-    uint64_t exp_at, floats;
+    uint64_t more_at, exp_at, floats;
 };
 RecordLayout record_layout(uint64_t m, uint64_t k) {
-    const uint64_t exp_at = m * (k / 128) * (kRecord / 4);
-    return {exp_at, exp_at + m};
+    const uint64_t records = m * (k / 128);
+    const uint64_t more_at = (records * kRecord + kPad) / 4, exp_at = more_at + records * (kMore / 4);
+    return {more_at, exp_at, exp_at + m};
 }
 
 template <int MT, int NT, int WM, int WN>
@@ -505,18 +618,18 @@ hipError_t run_gemm(Fp6Args& p, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Measured with [28672 x 4096], [4096 x 14336] and [4096 x 4096] at M = 20 to
-// 1024. Larger tiles read the activations' digits and the weights less often
-// per product (0.74 us per 32 x 256 outputs in 128 x 256 tiles, 0.81, 0.86 and
-// 1.04 in the others); smaller ones reach every CU with fewer rows.
-// [4096 x 14336] at M = 77: 39 us in 32 x 128 tiles and 8 slices, 204 in 64 x
-// 256 ones and one; at M = 1024 225 us in 64 x 256 and 4 slices, 201 in 128 x
-// 256 and 2; [4096 x 4096] at M = 512 48 us in 64 x 256 and 4 slices, 96 in 128
-// x 256 and one.
-constexpr GemmShape kShapes[] = {{128, 256, 1, {2.95f}},
-                                 {64, 256, 2, {1.8f, 2.9f}},
-                                 {32, 256, 2, {1.1f, 1.72f}},
-                                 {32, 128, 4, {0.7f, 1.1f, 1.6f, 2.07f}}};
+// Measured at k = 8192 with 1 to `most` blocks on every CU (3.75, 2.27 / 3.40,
+// 1.32 / 1.79, 0.88 / 1.16 / 1.76 / 2.22 us); the large tiles' full figures a
+// little lower, as whole products show them ([28672 x 4096] at M = 512 and 1024:
+// 3.2 and 2.94 us of two 64 x 256 blocks). Larger tiles read the activations'
+// digits and the weights less often per product; smaller ones reach every CU
+// with fewer rows. [4096 x 14336] at M = 200: 70 us in 32 x 256 tiles and 4
+// slices, 76 in 64 x 256 and 8; [4096 x 4096] at M = 200 33 us in 32 x 256 and 4,
+// 38 in 32 x 128 and one.
+constexpr GemmShape kShapes[] = {{128, 256, 1, {3.6f}},
+                                 {64, 256, 2, {2.27f, 3.3f}},
+                                 {32, 256, 2, {1.32f, 1.79f}},
+                                 {32, 128, 4, {0.88f, 1.16f, 1.76f, 2.22f}}};
 
 }  // namespace
 
@@ -542,8 +655,7 @@ bool qgemm_fp6_takes(const float* a, const QuantWeight* const* w, uint32_t nseg,
             return false;
         n += x.n;
     }
-    // byte offsets of the records in 32 bits
-    return m * (w[0]->k / 128) * kRecord <= 0xffffffffull && m * n <= 0xffffffffffull &&
+    return m * n <= 0xffffffffffull &&
            record_layout(m, w[0]->k).floats <= ws.floats;
 }
 
@@ -555,17 +667,19 @@ hipError_t launch_qgemm_fp6(const float* a, const QuantWeight* const* w, float* 
     if (gamma != nullptr && (u != nullptr || !qgemm_norm_takes(k, gamma))) return hipErrorNotSupported;
     const RecordLayout lay = record_layout(m, k);
     uint8_t* const records = reinterpret_cast<uint8_t*>(ws.data);
+    uint8_t* const more = reinterpret_cast<uint8_t*>(ws.data + lay.more_at);
     int* const row_exp = reinterpret_cast<int*>(ws.data + lay.exp_at);
     const uint32_t kk = static_cast<uint32_t>(k);
     const unsigned rows = static_cast<unsigned>(m);
-    if (k <= 4096) split_fp6<1><<<rows, 256, 0, s>>>(a, u, records, row_exp, kk, gamma, eps);
-    else if (k <= 8192) split_fp6<2><<<rows, 256, 0, s>>>(a, u, records, row_exp, kk, gamma, eps);
-    else if (k <= 16384) split_fp6<4><<<rows, 256, 0, s>>>(a, u, records, row_exp, kk, nullptr, 0.f);
-    else split_fp6<0><<<rows, 256, 0, s>>>(a, u, records, row_exp, kk, nullptr, 0.f);
+    if (k <= 4096) split_fp6<1><<<rows, 256, 0, s>>>(a, u, records, more, row_exp, kk, gamma, eps);
+    else if (k <= 8192) split_fp6<2><<<rows, 256, 0, s>>>(a, u, records, more, row_exp, kk, gamma, eps);
+    else if (k <= 16384) split_fp6<4><<<rows, 256, 0, s>>>(a, u, records, more, row_exp, kk, nullptr, 0.f);
+    else split_fp6<0><<<rows, 256, 0, s>>>(a, u, records, more, row_exp, kk, nullptr, 0.f);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     Fp6Args p{};
     p.records = records;
+    p.more = more;
     p.row_exp = row_exp;
     p.nseg = nseg;
     p.m = static_cast<uint32_t>(m);
@@ -581,7 +695,7 @@ hipError_t launch_qgemm_fp6(const float* a, const QuantWeight* const* w, float* 
     const uint64_t part_at = (lay.floats + 63) / 64 * 64;
     const GemmChoice best =
         choose_gemm(kShapes, n, nseg, m, p.sb_total, part_at < ws.floats ? ws.floats - part_at : 0,
-                    [](uint32_t) { return true; });
+                    [](uint32_t) { return true; }, 64);
     const size_t shape = best.shape;
     p.slices = best.slices;
     p.partial = p.slices > 1 ? ws.data + part_at : nullptr;

@@ -1,9 +1,9 @@
 """INT4 q-GEMM for many rows on the 6-bit matrix cores, against float64.
 
-Bound: a superblock of 128 k is five products summed in f32 (each within 2^-22
-of the magnitudes it adds) and one multiply-add, superblocks add in f32, and
-an activation keeps 24 bits below the largest of the 32 that share its
-exponent (here: of its superblock's 128).
+Bound: a superblock of 128 k is six or eight products summed in f32 (each
+within 2^-22 of the magnitudes it adds) and one multiply-add, superblocks add in
+f32, and an activation keeps 29 or 39 bits below the power of two above the
+largest of the 32 that share its exponent (half_units).
 """
 import numpy as np
 import pytest
@@ -14,11 +14,30 @@ from starlight_amd.ir import BufferRef, Op, QuantFormat, Value, ValueRole
 pytestmark = pytest.mark.gpu
 
 
-def weight(hip, n, k, group, r, codes=None):
+# lane l of a superblock's 128 k holds 16 (i / 4) + 4 l + i % 4, i < 32
+LANE_K = np.array([[16 * (i // 4) + 4 * l + i % 4 for i in range(32)] for l in range(4)])
+
+
+def half_units(a):
+    """Largest rounding of each element's digits: half a unit of 2^-29 of its
+    block's power of two, of 2^-39 where more than 16 of the 32 are nonzero and
+    below 2^-8 of it."""
+    m, k = a.shape
+    b = np.abs(a.astype(np.float64)).reshape(m, k // 128, 128)[:, :, LANE_K]
+    e = np.frexp(b.max(axis=3))[1][..., None]
+    further = ((b != 0) & (b < np.ldexp(1.0, e - 8))).sum(axis=3, keepdims=True) > 16
+    half = np.ldexp(0.5, e - np.where(further, 39, 29))
+    out = np.empty((m, k // 128, 128))
+    out[:, :, LANE_K] = half
+    return out.reshape(m, k)
+
+
+def weight(hip, n, k, group, r, codes=None, scales=None):
     """(ref, value, float64 weight) of a bound INT4 weight with codes -8..7."""
     if codes is None:
         codes = r.integers(-8, 8, (n, k)).astype(np.int8)
-    scales = r.uniform(0.001, 0.05, (n, k // group)).astype(np.float32)
+    if scales is None:
+        scales = r.uniform(0.001, 0.05, (n, k // group)).astype(np.float32)
     words = quant.pack_codes(codes, QuantFormat.INT4)
     pb, sb = hip.upload_new_u32(words), hip.upload_new_f32(scales.ravel())
     hip.bind_quantized(pb, sb, QuantFormat.INT4, group, n, k)
@@ -41,8 +60,7 @@ def run(hip, a, w):
 def assert_products(got, a, deq):
     a64 = a.astype(np.float64)
     m, k = a.shape
-    top = np.repeat(np.abs(a64).reshape(m, k // 128, 128).max(axis=2), 128, axis=1)
-    bound = (k / 128 + 8) * 2.0**-22 * (np.abs(a64) @ np.abs(deq).T) + 2.0**-25 * (top @ np.abs(deq).T)
+    bound = (k / 128 + 8) * 2.0**-22 * (np.abs(a64) @ np.abs(deq).T) + half_units(a) @ np.abs(deq).T
     diff = np.abs(got.astype(np.float64) - a64 @ deq.T)
     assert np.all(diff <= bound + 1e-37), float(np.max(diff - bound))
 
@@ -76,6 +94,57 @@ def test_elements_far_below_their_row_keep_their_bits(hip):
     w = weight(hip, n, k, 128, r, codes)
     got = run(hip, a, w)
     assert_products(got, a[:, 128:], w[2][:, 128:])
+
+
+def outliers(r, m, k, factor, channels):
+    a = r.standard_normal((m, k)).astype(np.float32)
+    at = {"one": np.arange(77, 78), "each 32": np.arange(7, k, 32),
+          "8 of 32": np.flatnonzero(np.arange(k) % 128 % 16 < 4)}[channels]
+    a[:, at] *= np.float32(factor)
+    return a, at
+
+
+# Channels far above the others, under zero codes: the others' products keep the
+# precision that 22 bits of each element give (2^-22 normwise), as with each
+# element split into two fp16 parts. k: rows held by the threads, and longer.
+@pytest.mark.parametrize("factor", [30, 1e3, 1e4, 1e5])
+@pytest.mark.parametrize("channels", ["one", "each 32", "8 of 32"])
+@pytest.mark.parametrize("m,n,k", [(33, 70, 512), (100, 40, 4096), (17, 20, 16512), (130, 300, 256)])
+def test_outlier_channels(hip, m, n, k, factor, channels):
+    r = np.random.default_rng(k + m)
+    a, at = outliers(r, m, k, factor, channels)
+    codes = r.integers(-8, 8, (n, k)).astype(np.int8)
+    codes[:, at] = 0
+    w = weight(hip, n, k, 128, r, codes)
+    got = run(hip, a, w)
+    want = a.astype(np.float64) @ w[2].T
+    assert np.linalg.norm(got - want) <= 2.0**-22 * np.linalg.norm(want)
+
+
+# Each column one code of 1 under a scale of 1: the activations themselves as the
+# digits hold them. Joined from the lowest on, each sum rounds by 2^-24 of itself:
+# the last one is the value, the one before at most 16/31 of the highest nonzero
+# digit's unit, which is at most 16/15 of the value, the others 1/32 of that.
+@pytest.mark.parametrize("kind", ["normal", "silu", "one", "each 32", "8 of 32", "spread", "denormal"])
+def test_activations_as_their_digits(hip, kind):
+    r = np.random.default_rng(14)
+    m, k = 49, 256
+    if kind == "normal":
+        a = r.standard_normal((m, k))
+    elif kind == "silu":
+        g = 3 * r.standard_normal((m, k))
+        a = g / (1 + np.exp(-g)) * r.standard_normal((m, k))
+    elif kind == "spread":
+        a = np.ldexp(r.uniform(-1, 1, (m, k)), r.integers(-60, 60, (m, k)))
+        a[r.random((m, k)) < 0.2] = 0
+    elif kind == "denormal":
+        a = np.ldexp(r.uniform(-1, 1, (m, k)), -122 - r.integers(0, 20, (m, k)))
+    else:
+        a = outliers(r, m, k, 2e3, kind)[0]
+    a = a.astype(np.float32)
+    w = weight(hip, k, k, 128, r, np.eye(k, dtype=np.int8), np.ones((k, 2), np.float32))
+    got = run(hip, a, w).astype(np.float64)
+    assert np.all(np.abs(got - a) <= 2.2 * 2.0**-24 * np.abs(a) + half_units(a) + 2.0**-149)
 
 
 @pytest.mark.parametrize("scale", [1e-42, 1e-37, 1e30, 3e37])
