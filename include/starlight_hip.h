@@ -197,14 +197,17 @@ sl_status sl_hip_dispatch(sl_hip_device *device, const sl_op *op, const sl_buffe
  * as sl_hip_dispatch does, then enqueues this one command's kernels on the
  * device's stream at once (no fusion, no graph, past_len taken from the
  * scalar), and calls no hipMalloc, hipFree or allocating routine. Its
- * scratch memory (attention partials, SwiGlu intermediates, split-K
- * partials) is a static array of SL_HIP_STATIC_SCRATCH_BYTES held by each
- * GPU the library runs on until the process ends, not the device workspace.
+ * scratch memory (decode attention partials, SwiGlu intermediates, the
+ * normalised rows of RmsNormMatMul, and the partials and split activations of
+ * quantized products) is a static array of SL_HIP_STATIC_SCRATCH_BYTES held by
+ * each GPU the library runs on until the process ends, not the device
+ * workspace. The other commands (a dense MatMulNT and a prompt's attention
+ * among them) use none of it.
  * Errors: Execution when commands are still logged (call sl_hip_submit
  * first) or the array's address could not be found at device creation;
  * Unimplemented when the command needs more scratch than the array holds.
- * Every call on one GPU shares that GPU's array: calls that overlap on one
- * GPU (several devices or streams on it) race. A Gather whose id buffer is
+ * Every call on one GPU shares that GPU's array: calls of the commands named
+ * that overlap on one GPU (several devices or streams on it) race. A Gather whose id buffer is
  * larger than 16 MiB checks its ids with a device-to-host copy and a stream
  * synchronize, which graph capture does not allow. */
 #define SL_HIP_STATIC_SCRATCH_BYTES (16u << 20)

@@ -1528,7 +1528,7 @@ sl_status sl_hip_dispatch_noalloc(sl_hip_device* d, const sl_op* op, const sl_bu
     // past_len reaches the kernels as the scalar itself (no device word)
     const hipError_t e =
         slhip::launch(d, plan, inputs, &out, nullptr,
-                      slhip::Workspace{d->static_scratch, slhip::kStaticScratchFloats});
+                      slhip::Workspace{d->static_scratch, slhip::kStaticScratchFloats, true});
     if (e != hipSuccess) return d->hip_fail(e);
     return SL_OK;
 }

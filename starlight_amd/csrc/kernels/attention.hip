@@ -1476,7 +1476,8 @@ hipError_t run_prefill(const AttentionArgs& a, const Geo& g, const Workspace& ws
     const uint64_t tiles = (a.max_seq + 63) / 64 * 2;  // an even count: stages are two tiles
     const uint64_t words = a.batch * a.kv_heads * tiles * (wide ? plane_words<128>() : plane_words<64>());
     const uint64_t flag_floats = (a.batch * a.kv_heads * tiles + 63) / 64 * 64, floats = flag_floats + 4 * words;
-    if (a.seq < (wide ? 256 : 512) || !(a.scale >= 0.f && a.scale <= 32.f) || tiles > 0xffffffull || keep + floats + 64 > ws.floats) {
+    if (a.seq < (wide ? 256 : 512) || !(a.scale >= 0.f && a.scale <= 32.f) || tiles > 0xffffffull || ws.shared ||
+        keep + floats + 64 > ws.floats) {
         if (wide) attn_prefill<128, 2><<<grid, 512, 0, s>>>(g, qtiles);
         else attn_prefill<64, 2><<<grid, 512, 0, s>>>(g, qtiles);
         return hipGetLastError();

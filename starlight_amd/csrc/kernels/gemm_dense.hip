@@ -195,7 +195,7 @@ hipError_t launch_gemm_dense(const GemvDense& f, const Workspace& ws, hipStream_
     const uint64_t tiles = static_cast<uint64_t>(p.rows) * p.cols;
     float best = INFINITY;
     for (uint32_t z = 1; z <= 16 && z <= stages; z *= 2) {
-        if (z > 1 && z * p.slice_floats > ws.floats) break;
+        if (z > 1 && (ws.shared || z * p.slice_floats > ws.floats)) break;
         const uint64_t per_cu = (tiles * z + compute_units() - 1) / compute_units();
         float t = static_cast<float>(per_cu * ((stages + z - 1) / z) * mt) * 0.25f;
         if (z > 1) t += 3.5f + static_cast<float>(p.slice_floats * (2 * z + 1)) * 1e-6f;

@@ -14,6 +14,9 @@ namespace slhip {
 struct Workspace {
     float* data;
     uint64_t floats;
+    // Other calls on this GPU may be using it at the same time: left alone by
+    // kernels that only run faster with it (dense k slices, split K and V).
+    bool shared = false;
 
     // The part of `data` after the first `used` floats.
     Workspace after(uint64_t used) const {

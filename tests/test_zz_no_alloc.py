@@ -12,7 +12,7 @@ import pytest
 
 from conftest import assert_normwise
 from starlight_amd import quant
-from starlight_amd.device import DeviceError
+from starlight_amd.device import DeviceError, HipDevice
 from starlight_amd.ir import BufferRef, Op, QuantFormat, Value, ValueRole
 
 pytestmark = pytest.mark.gpu
@@ -111,6 +111,33 @@ def test_rms_norm_matmul_twice_second_smaller(hip):
         gamma = np.random.default_rng(seed + 1).uniform(0.5, 1.5, hidden).astype(np.float32)
         run_weighted(hip, Op.rms_norm_matmul(1e-5), x, Value.f32([rows, hidden]), [w], [gamma], rows * out_f,
                      Value.f32([rows, out_f]))
+
+
+def test_commands_without_scratch_leave_the_shared_array_alone(hip, monkeypatch):
+    """A dense product and a prompt's attention, which a device with a workspace
+    runs in k slices and on split K and V, take the forms of one without room
+    here: calls of them that overlap on a GPU do not meet in its array."""
+    r = np.random.default_rng(9)
+    m, k, n = 200, 8192, 256
+    a, w = r.uniform(-1, 1, m * k).astype(np.float32), r.uniform(-1, 1, n * k).astype(np.float32)
+    H, S, D, max_seq = 2, 520, 64, 576
+    q, kn, v = (r.standard_normal(h * S * D).astype(np.float32) for h in (H, 1, 1))
+    cache = np.zeros(2 * max_seq * D, np.float32)
+    q4, k4 = Value.f32([1, H, S, D]), Value.f32([1, 1, S, D])
+    cases = [(Op.matmul_nt(), [a, w], [Value.f32([m, k]), Value.f32([n, k])], m * n, Value.f32([m, n]), ()),
+             (Op.causal_attention(0, H, 1, D, 0.125), [q, kn, v, cache],
+              [q4, k4, k4, Value.f32([1, 1, 2, max_seq, 1, D], ValueRole.STATE)], q.size, q4, [0])]
+    monkeypatch.setenv("SL_HIP_WORKSPACE_BYTES", "65536")
+    small = HipDevice(0)
+    try:
+        for op, inputs, vals, out_len, out_val, scalars in cases:
+            bare, _ = run_both(small, op, inputs, vals, out_len, out_val, scalars)
+            (full, _), (noalloc, _) = run_both(hip, op, inputs, vals, out_len, out_val, scalars)
+            np.testing.assert_array_equal(noalloc, bare[0])
+            assert not np.array_equal(full, bare[0])  # the form with room is another one
+            assert_normwise(full, bare[0])
+    finally:
+        small.close()
 
 
 def test_rejects_logged_commands_and_oversized_scratch(hip):
