@@ -1030,9 +1030,10 @@ size_t try_fuse_attention(Device* d, size_t i, hipError_t* err) {
     const Workspace ws{d->workspace, d->workspace_floats};
     const uint64_t mirror_at = (attention_fused_workspace_floats(a) + 63) / 64 * 64;
     // The output projection is chained (it reads the mirror, not MergeHeads'
-    // output) only for decode (at most 16 rows, the fused GEMV's) and when
-    // the mirror fits; otherwise it runs on its own and reads MergeHeads'
-    // output, which must then be written.
+    // output) only for decode (at most 16 rows, the fused GEMV's, and not the
+    // prefill form, which a 16-token prompt takes and which writes no mirror)
+    // and when the mirror fits; otherwise it runs on its own and reads
+    // MergeHeads' output, which must then be written.
     const Logged* mm = mh && i + used < n ? &d->log[i + used] : nullptr;
     GemvDense dense{};  // the same for a dense weight
     if (mm && mm->plan.code == SL_OP_MATMUL_NT && !mm->plan.quant[1].present && mm->plan.batch_b == 1 &&
@@ -1049,7 +1050,8 @@ size_t try_fuse_attention(Device* d, size_t i, hipError_t* err) {
     const bool dense_chain = gemv_dense_takes(dense);
     const bool chain = mm && mm->plan.code == SL_OP_MATMUL_NT && same_ref(mm->in[0], mh->out) &&
                        (mfma_weight(d, *mm, 1) || dense_chain) && mm->plan.batch * mm->plan.m == B * S &&
-                       mm->plan.k == H * D && B * S <= 16 && mirror_at + B * S * H * D <= ws.floats;
+                       mm->plan.k == H * D && B * S <= 16 && !attention_fused_prefill(a) &&
+                       mirror_at + B * S * H * D <= ws.floats;
     const bool merged_needed = mh != nullptr && !dead_after(d, i + used, mh->out, chain ? i + used : SIZE_MAX);
     // outputs of the merge kernel: no overlap with the cache, or with each other
     if (overlaps(att, cache_ref) || (mh && overlaps(mh->out, cache_ref)) ||
