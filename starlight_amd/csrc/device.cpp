@@ -37,6 +37,7 @@
 #include <utility>
 #include <vector>
 
+#include "arena.h"
 #include "kernels/kernels.h"
 #include "internal.h"
 #include "plan.h"
@@ -59,9 +60,9 @@ struct Buffer {
     bool mirrored = false;
     // group-quantized binding
     uint32_t scales = 0;
-    uint8_t* tiles = nullptr;  // private codes, then (Mfma) tile-ordered scales
+    uint8_t* tiles = nullptr;  // private codes, then (Mfma) tile-ordered scales (Device::tile_memory)
     float* tile_scales = nullptr;
-    uint8_t* fp6 = nullptr;  // 6-bit copy (its own allocation), where the weight has one
+    uint8_t* fp6 = nullptr;  // 6-bit copy (Device::fp6_memory), where the weight has one
     QuantLayout layout = QuantLayout::RowMajor;
 };
 
@@ -91,6 +92,7 @@ struct Device : BufferView {
     int ordinal = 0;
     hipStream_t stream = nullptr;
     std::vector<Buffer> buffers;
+    Arena tile_memory, fp6_memory;  // the quantized weights' private copies
     float* workspace = nullptr;
     uint64_t workspace_floats = 0;
     float* static_scratch = nullptr;  // this GPU's static array (no-allocation entry point)
@@ -1451,9 +1453,9 @@ void sl_hip_device_destroy(sl_hip_device* d) {
     if (d->dyn) (void)hipFree(d->dyn);
     for (auto& b : d->buffers) {
         if (b.base) (void)hipFree(b.base);
-        if (b.tiles) (void)hipFree(b.tiles);
-        if (b.fp6) (void)hipFree(b.fp6);
     }
+    d->tile_memory.clear();
+    d->fp6_memory.clear();
     if (d->workspace) (void)hipFree(d->workspace);
     if (d->rope_tab) (void)hipFree(d->rope_tab);
     (void)hipStreamDestroy(d->stream);
@@ -1718,26 +1720,21 @@ sl_status sl_hip_bind_quantized(sl_hip_device* d, uint32_t payload, uint32_t sca
     const uint64_t bytes = scale_floats ? scale_offset + scale_floats * 4 : code_bytes;
     if (pb.tiles) {
         (void)hipStreamSynchronize(d->stream);
-        (void)hipFree(pb.tiles);
-        if (pb.fp6) (void)hipFree(pb.fp6);
+        d->tile_memory.give(pb.tiles);
+        d->fp6_memory.give(pb.fp6);
+        pb.desc.quantized = 0;  // should the new copy find no room
         pb.tiles = nullptr;
         pb.tile_scales = nullptr;
         pb.fp6 = nullptr;
     }
     if (bytes != 0) {
-        if (hipMalloc(reinterpret_cast<void**>(&pb.tiles), bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            pb.tiles = nullptr;
-            return d->fail(Error::out_of_memory(bytes / 4));
-        }
+        pb.tiles = static_cast<uint8_t*>(d->tile_memory.take(bytes));
+        if (pb.tiles == nullptr) return d->fail(Error::out_of_memory(bytes / 4));
         if (scale_floats) pb.tile_scales = reinterpret_cast<float*>(pb.tiles + scale_offset);
     }
     // without room for the 6-bit copy, many rows take the fp16 route
     const uint64_t fp6_bytes = slhip::quant_fp6_bytes(qformat, n, k, group_size, layout);
-    if (fp6_bytes != 0 && hipMalloc(reinterpret_cast<void**>(&pb.fp6), fp6_bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        pb.fp6 = nullptr;
-    }
+    if (fp6_bytes != 0) pb.fp6 = static_cast<uint8_t*>(d->fp6_memory.take(fp6_bytes));
     pb.desc.quantized = 1;
     pb.desc.qformat = qformat;
     pb.desc.group_size = group_size;
