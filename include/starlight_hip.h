@@ -162,7 +162,9 @@ typedef struct sl_hip_device sl_hip_device;
 /* CpuDevice::new() (device.rs:41-45). Opens HIP device `ordinal`, creates the
  * device's stream and its fixed workspace (512 MiB, or the byte count in the
  * environment variable SL_HIP_WORKSPACE_BYTES, at least 64 KiB; fused
- * launches that do not fit a smaller workspace run unfused). */
+ * launches that do not fit a smaller workspace run unfused). With
+ * SL_HIP_FP6_COPIES=0 in the environment, sl_hip_bind_quantized makes no 6-bit
+ * copies. */
 sl_status sl_hip_device_create(int ordinal, sl_hip_device **out);
 void sl_hip_device_destroy(sl_hip_device *device);
 
@@ -237,8 +239,15 @@ void sl_hip_last_error(const sl_hip_device *device, sl_error *out);
  * SL_ENCODING_GROUPWISE_QUANTIZED (role Param, dtype F32, logical shape
  * [n, k]) reads the payload through a BufferRef { payload, 0, words }.
  * Ports that accept it: MatMulNT B, SwiGlu gate/up/down, RmsNormMatMul matrix.
- * The device repacks the codes into a private tile layout here; a later
- * upload_u32 to the payload buffer refreshes that copy. */
+ * The device repacks the codes into a private tile layout here (as many bytes
+ * again as the payload and scales); a later upload_u32 to the payload buffer
+ * refreshes that copy. An INT4 weight whose group_size is a multiple of 128
+ * gets a second one, in 6-bit codes (0.75 bytes a weight, 6.0 GB at 8B), which
+ * products of more than 16 rows read: without it they take 1.3 to 3 times as
+ * long. Where memory runs out, on this call or a later allocation of the same
+ * device, the device gives up all its 6-bit copies first and makes no new ones;
+ * memory that something else allocates is not seen, so a program that needs the
+ * room for that declines them (SL_HIP_FP6_COPIES, above). */
 sl_status sl_hip_bind_quantized(sl_hip_device *device, uint32_t payload, uint32_t scales,
                                 uint32_t qformat, uint32_t group_size, uint32_t n, uint32_t k);
 

@@ -93,6 +93,7 @@ struct Device : BufferView {
     hipStream_t stream = nullptr;
     std::vector<Buffer> buffers;
     Arena tile_memory, fp6_memory;  // the quantized weights' private copies
+    bool fp6_copies = true;         // whether weights bound now get a 6-bit copy
     float* workspace = nullptr;
     uint64_t workspace_floats = 0;
     float* static_scratch = nullptr;  // this GPU's static array (no-allocation entry point)
@@ -143,6 +144,25 @@ struct Device : BufferView {
 namespace {
 
 sl_status flush(Device* d);
+void drop_graphs(Device* d);
+
+// Called where `bytes` of device memory were not to be had. The 6-bit copies
+// only make many rows faster, so they go first: true if there were any, and the
+// allocation is worth another try. Logged commands take their weights as they
+// are when submitted; captured graphs hold the copies' addresses.
+bool make_room(Device* d, uint64_t bytes) {
+    size_t free = 0, total = 0;
+    if (d->fp6_memory.empty() || hipMemGetInfo(&free, &total) != hipSuccess || bytes > total) {
+        (void)hipGetLastError();
+        return false;
+    }
+    (void)hipStreamSynchronize(d->stream);
+    drop_graphs(d);
+    for (Buffer& b : d->buffers) b.fp6 = nullptr;
+    d->fp6_memory.clear();
+    d->fp6_copies = false;
+    return true;
+}
 
 float* fptr(Device* d, const sl_buffer_ref& r) {
     return static_cast<float*>(d->buffers[r.buffer].ptr) + r.offset;
@@ -164,9 +184,9 @@ sl_status allocate(Device* d, size_t elements, size_t align, uint32_t kind, uint
     if (elements != 0) {
         const size_t bytes = elements * 4;
         const size_t extra = align > 256 ? align : 0;  // hipMalloc returns 256-byte aligned memory
-        if (hipMalloc(&b.base, bytes + extra) != hipSuccess) {
+        while (hipMalloc(&b.base, bytes + extra) != hipSuccess) {
             (void)hipGetLastError();
-            return d->fail(Error::out_of_memory(elements));
+            if (!make_room(d, bytes + extra)) return d->fail(Error::out_of_memory(elements));
         }
         uintptr_t p = reinterpret_cast<uintptr_t>(b.base);
         if (extra) p = (p + align - 1) & ~static_cast<uintptr_t>(align - 1);
@@ -1423,6 +1443,8 @@ sl_status sl_hip_device_create(int ordinal, sl_hip_device** out) {
         return SL_ERR_OUT_OF_MEMORY;
     }
     d->workspace_floats = ws_bytes / 4;
+    const char* const fp6 = std::getenv("SL_HIP_FP6_COPIES");
+    d->fp6_copies = fp6 == nullptr || std::strcmp(fp6, "0") != 0;
     if (hipMalloc(reinterpret_cast<void**>(&d->rope_tab), slhip::kRopeTableFloats * 4) != hipSuccess ||
         hipMalloc(reinterpret_cast<void**>(&d->dyn), slhip::kLogFlushLength * sizeof(uint32_t)) != hipSuccess) {
         (void)hipGetLastError();
@@ -1728,12 +1750,14 @@ sl_status sl_hip_bind_quantized(sl_hip_device* d, uint32_t payload, uint32_t sca
         pb.fp6 = nullptr;
     }
     if (bytes != 0) {
-        pb.tiles = static_cast<uint8_t*>(d->tile_memory.take(bytes));
+        do {
+            pb.tiles = static_cast<uint8_t*>(d->tile_memory.take(bytes));
+        } while (pb.tiles == nullptr && slhip::make_room(d, bytes));
         if (pb.tiles == nullptr) return d->fail(Error::out_of_memory(bytes / 4));
         if (scale_floats) pb.tile_scales = reinterpret_cast<float*>(pb.tiles + scale_offset);
     }
     // without room for the 6-bit copy, many rows take the fp16 route
-    const uint64_t fp6_bytes = slhip::quant_fp6_bytes(qformat, n, k, group_size, layout);
+    const uint64_t fp6_bytes = d->fp6_copies ? slhip::quant_fp6_bytes(qformat, n, k, group_size, layout) : 0;
     if (fp6_bytes != 0) pb.fp6 = static_cast<uint8_t*>(d->fp6_memory.take(fp6_bytes));
     pb.desc.quantized = 1;
     pb.desc.qformat = qformat;

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from starlight_amd import quant
+from starlight_amd.device import HipDevice
 from starlight_amd.ir import BufferRef, Op, QuantFormat, Value, ValueRole
 
 pytestmark = pytest.mark.gpu
@@ -199,6 +200,29 @@ def test_infinities_and_nan_stay_in_their_row(hip):
     assert np.all(np.isnan(got[bad]))
     keep = [i for i in range(40) if i not in bad]
     assert_products(got[keep], a[keep], w[2])
+
+
+# A device that made no 6-bit copies: the fp16 route, which keeps 22 bits of an
+# element down to 2^-40 of its row's largest, whose superblock is 8 products summed
+# in f32, and which sums in slices for one weight and for several
+@pytest.mark.parametrize("m,n,k,group", [(17, 33, 128, 128), (64, 129, 1152, 128), (65, 260, 4096, 4096),
+                                         (77, 128, 14336, 128), (129, 16, 8320, 128), (300, 520, 512, 256),
+                                         (520, 4100, 256, 128)])
+def test_products_without_the_copies(monkeypatch, m, n, k, group):
+    monkeypatch.setenv("SL_HIP_FP6_COPIES", "0")
+    dev = HipDevice(0)
+    try:
+        r = np.random.default_rng(m + n + k)
+        a = (r.standard_normal((m, k)) * 10.0 ** r.uniform(-6, 3, (m, 1))).astype(np.float32)
+        a[3] = 0.0
+        w = weight(dev, n, k, group, r)
+        got = run(dev, a, w)
+        a64 = np.abs(a.astype(np.float64))
+        bound = ((k / 128 + 8) * 2.0**-21 * a64 + 2.0**-40 * a64.max(axis=1, keepdims=True)) @ np.abs(w[2]).T
+        assert np.all(np.abs(got.astype(np.float64) - a.astype(np.float64) @ w[2].T) <= bound)
+        test_norm_and_three_projections_in_slices(dev, 77, 4096, (300, 129, 65))
+    finally:
+        dev.close()
 
 
 def test_reuploaded_payload_and_scales_refresh_the_copy(hip):

@@ -6,8 +6,8 @@ import numpy as np
 import pytest
 
 from starlight_amd import quant
-from starlight_amd.device import HipDevice, load_library
-from starlight_amd.ir import QuantFormat
+from starlight_amd.device import DeviceError, HipDevice, load_library
+from starlight_amd.ir import BufferRef, Op, QuantFormat, Value
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,67 @@ def test_copies_are_given_back():
         bind(dev, 14336, 4096, QuantFormat.INT4)
     dev.close()
     assert free_bytes() >= before - (4 << 20)
+
+
+N, K, M = 512, 1024, 48
+
+
+def products(dev, weight, words, a, times=1):
+    out = dev.allocate_f32(M * N, 256)
+    ab = dev.upload_new_f32(a)
+    for _ in range(times):  # (the third is a captured graph's)
+        dev.dispatch(Op.matmul_nt(), [BufferRef(ab, 0, M * K), BufferRef(weight, 0, words)],
+                     [Value.f32([M, K]), Value.quantized([N, K], QuantFormat.INT4, 128)],
+                     [BufferRef(out, 0, M * N)], [Value.f32([M, N])])
+        dev.submit()
+    return dev.read_f32(out, M * N)
+
+
+def inputs():
+    r = np.random.default_rng(3)
+    words, scales = quant.quantize((r.standard_normal((N, K)) * 0.05).astype(np.float32), 128, QuantFormat.INT4)
+    return words, scales, r.standard_normal(M * K).astype(np.float32)
+
+
+def bound(dev, words, scales):
+    return bind(dev, N, K, QuantFormat.INT4, dev.upload_new_u32(words), dev.upload_new_f32(scales))[0]
+
+
+def test_copies_can_be_declined(monkeypatch):
+    """Without the 6-bit copies the same products come from the fp16 route."""
+    words, scales, a = inputs()
+    results, used = [], []
+    for decline in (False, True):
+        if decline:
+            monkeypatch.setenv("SL_HIP_FP6_COPIES", "0")
+        dev = HipDevice(0)
+        before = free_bytes()
+        results.append(products(dev, bound(dev, words, scales), words.size, a))
+        used.append(before - free_bytes())
+        dev.close()
+    assert used[1] < used[0]
+    assert not np.array_equal(results[0], results[1])
+    assert np.linalg.norm(results[0] - results[1]) <= 2.0**-21 * np.linalg.norm(results[0])
+
+
+def test_a_failing_allocation_takes_the_6_bit_copies_back(monkeypatch):
+    """An allocation of the whole GPU fails with and without them, but they are
+    gone then, nothing else is, and later products are the fp16 route's."""
+    words, scales, a = inputs()
+    monkeypatch.setenv("SL_HIP_FP6_COPIES", "0")
+    dev = HipDevice(0)
+    without = products(dev, bound(dev, words, scales), words.size, a)
+    dev.close()
+    monkeypatch.delenv("SL_HIP_FP6_COPIES")
+    dev = HipDevice(0)
+    weight = bound(dev, words, scales)
+    assert not np.array_equal(products(dev, weight, words.size, a, 3), without)
+    free, total = memory()
+    with pytest.raises(DeviceError) as e:
+        dev.allocate_f32(total // 4, 256)
+    assert e.value == DeviceError.out_of_memory(total // 4)
+    assert free_bytes() > free
+    assert np.array_equal(products(dev, weight, words.size, a, 3), without)
+    # bound later: no copy either
+    assert np.array_equal(products(dev, bound(dev, words, scales), words.size, a), without)
+    dev.close()
