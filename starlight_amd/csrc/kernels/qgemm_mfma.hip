@@ -1,6 +1,7 @@
 // Group-quantized MatMulNT for many activation rows (prefill):
 // out[m, n] = sum_k a[m, k] * (q[n, k] * s[n, k / G]), on the fp16 matrix
-// cores, from the Mfma tile layout of the weights.
+// cores, from the Mfma tile layout of the weights. INT4 weights that have a 6-bit
+// copy (groups of whole superblocks) take qgemm_fp6.hip where its activations fit.
 //
 // Exactness plan. The codes q are small integers, exact in fp16. Each
 // activation row is scaled by 2^(15 - E) (|a| < 2^E over the row, so the
@@ -23,7 +24,8 @@
 //  * qgemm_mfma: 128 x 128 output tiles, 4 waves of 64 x 64 (4 x 4 MFMA
 //    tiles of 16 x 16), k in stages of 32 through double-buffered LDS; or
 //    64 x 128 tiles (waves of 32 x 64) in stages of 32 or 64; a grid z of
-//    2 cuts k in two slices whose partial sums slices_sum adds. The
+//    2, 4 or 8 cuts k in as many slices, of one weight or several, whose
+//    partial sums slices_sum adds. The
 //    weight stage is read from the tile layout (per 16-row tile and 128-k
 //    superblock; a 32-k stage is half of one 64-k half: 32 lanes x 8 bytes
 //    for INT4, x 16 bytes for INT8) and converted to fp16 codes in LDS

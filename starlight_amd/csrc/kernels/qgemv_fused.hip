@@ -865,10 +865,11 @@ hipError_t launch_qgemv_fused(const QgemvFused& f, hipStream_t s) {
 #define SL_QGEMV_FUSED_G(B, T) \
     (spg == 1 ? SL_QGEMV_FUSED(B, T, 1) : spg == 2 ? SL_QGEMV_FUSED(B, T, 2) : SL_QGEMV_FUSED(B, T, 0))
     if (slices > 1) {
-        // k slices: 16 waves, 8 float4 per thread. (Three or four rows in the
-        // form for up to four, not on the split-k fallback with its own
-        // reduction and Add: INT8 [4096 x 14336] at M = 4, two 8B layers
-        // decoding for four sequences 584 -> 519 us over two steps.)
+        // k slices: 16 waves, 8 float4 per thread. (Up to four rows (one from
+        // k = 32768 on, two from 16384) in the form for as many, not on the
+        // split-k fallback with its own reduction and Add: INT8 [4096 x 14336]
+        // at M = 4, two 8B layers decoding for four sequences 584 -> 519 us
+        // over two steps.)
         if (f4 > 8) return hipErrorNotSupported;
 #define SL_QGEMV_SLICED_LR(B, G, L) \
     qgemv_fused<B, 1, G, L, 8, 16, true, kSmStream><<<grid, threads, lds, s>>>(f.a, f.gamma, mk, p.k, p)

@@ -1,4 +1,4 @@
-"""Quantized MatMulNT of 3 and 4 rows whose activations exceed the fused
+"""Quantized MatMulNT of 1 to 4 rows whose activations exceed the fused
 GEMV's LDS (m * k > 32768): k in slices, in the kernel's form for up to four
 rows, against float64. The limbs keep 22 bits below a 256-element chunk's
 maximum and the groups' sums add in f32: (k / 64 + 8) roundings of 2^-22."""
@@ -13,8 +13,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("fmt", [QuantFormat.INT4, QuantFormat.INT8])
 @pytest.mark.parametrize("m,k,n,group", [(3, 14336, 300, 128), (4, 14336, 33, 64), (4, 8448, 520, 128),
-                                         (3, 11008, 64, 64), (4, 16384, 17, 256), (4, 28672, 48, 128)])
-def test_three_and_four_rows_in_slices(hip, fmt, m, k, n, group):
+                                         (3, 11008, 64, 64), (4, 16384, 17, 256), (4, 28672, 48, 128),
+                                         (1, 33024, 300, 128), (1, 57344, 33, 64), (2, 16640, 520, 128),
+                                         (2, 28672, 130, 64), (2, 32768, 17, 512)])
+def test_up_to_four_rows_in_slices(hip, fmt, m, k, n, group):
     r = np.random.default_rng(m + n + k)
     x = (r.standard_normal((m, k)) * 10.0 ** r.uniform(-4, 3, (m, 1))).astype(np.float32)
     top = 8 if fmt == QuantFormat.INT4 else 128
