@@ -33,6 +33,7 @@ struct Workspace {
 // loads one at the first use of any of its kernels); preload_code loads
 // them all and returns the first error.
 hipError_t load_code_attention();
+hipError_t load_code_attention_bf16();
 hipError_t load_code_elementwise();
 hipError_t load_code_gemm_dense();
 hipError_t load_code_gemv_dense();
@@ -43,6 +44,7 @@ hipError_t load_code_qgemm_fp6();
 hipError_t load_code_qgemm_mfma();
 hipError_t load_code_qgemv_fused();
 hipError_t load_code_qgemv_mfma();
+hipError_t load_code_qgemv_sliced();
 hipError_t load_code_qmatmul();
 hipError_t load_code_rope();
 hipError_t load_code_slices();
@@ -51,7 +53,8 @@ inline hipError_t preload_code() {
                                      load_code_matmul,    load_code_norm_softmax, load_code_qgemm_mfma,
                                      load_code_qgemv_fused, load_code_qgemv_mfma, load_code_qmatmul,
                                      load_code_rope,      load_code_gemv_dense, load_code_qgemm_fp6,
-                                     load_code_gemm_dense, load_code_slices};
+                                     load_code_gemm_dense, load_code_slices, load_code_attention_bf16,
+                                     load_code_qgemv_sliced};
     hipError_t first = hipSuccess;
     for (auto load : loads) {
         const hipError_t e = load();
@@ -165,6 +168,11 @@ uint64_t attention_workspace_floats(const AttentionArgs& a);
 // workspace floats its kernels use before any caller area: the decode
 // partials, or the prefill form's rotated q.
 bool attention_fused_prefill(const AttentionArgs& a);
+// The prefill attention of prepared q on the bf16 matrix cores, over a cache that
+// holds the chunk's keys (attention_bf16.hip); hipErrorNotSupported, nothing
+// launched, for chunks that the f32 form takes.
+hipError_t launch_attention_prefill_bf16(const AttentionArgs& a, const float* q, const Workspace& ws, uint64_t keep,
+                                         hipStream_t s);
 uint64_t attention_fused_workspace_floats(const AttentionArgs& a);
 
 // Decode attention over a paged KV cache (one new token per row): row b has

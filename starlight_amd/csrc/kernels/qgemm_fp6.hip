@@ -37,9 +37,9 @@
 // 1024 238 against 304 (213), M = 512 130 against 186 (117), M = 77 46 against
 // 159 (41); [4096 x 4096] M = 77 26 against 56 (25). What bounds it now: vector
 // and matrix instructions of a SIMD's waves do not overlap here, and a 64 x 256
-// tile's pass has 96 products (1,536 cycles) and about 170 vector instructions
-// (680) per wave, two waves per SIMD: 4,430 of about 6,500 cycles measured; LDS
-// is busy for 2,950 of them (reads of the digits, and the stage's writes in the
+// tile's pass has 96 products (1,536 cycles) and 178 vector instructions (712)
+// per wave, two waves per SIMD: 4,500 of 5,830 cycles measured (at 1.9 GHz); LDS
+// is busy for 2,370 of them (reads of the digits, and the stage's writes in the
 // middle of the pass: at its end, 1-2% slower; loads straight into LDS the same
 // time as through registers). Deeper operand prefetch and wave priorities
 // changed nothing, and gathering the records in operand order from memory (no
@@ -58,9 +58,10 @@
 //    x 16 then 4 x 8 bytes, and four block scales with the flag of further
 //    digits, which lie in planes of their own;
 //  * qgemm_fp6: a block's rows of a superblock, contiguous, staged through LDS
-//    as they are (592 bytes a row: the 16 rows of one operand read fall on
-//    disjoint groups of 4 banks), shared by the block's waves; weights straight
-//    from memory into registers, one superblock ahead.
+//    as they are (592 bytes a row: the 16 rows of one operand read begin 20
+//    banks apart, no two on the same 4; rows of 640 bytes: 400 -> 480 us), shared
+//    by the block's waves; weights straight from memory into registers, one
+//    superblock ahead.
 #include "common.h"
 #include "kernels.h"
 #include "qgemm_act.h"

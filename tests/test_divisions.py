@@ -1,5 +1,5 @@
 """The q-GEMV's multiply-shift divisions are exact over the ranges its
-launcher lets through (starlight_amd/csrc/kernels/qgemv_fused.hip, Args and
+launcher lets through (starlight_amd/csrc/kernels/qgemv_kernel.h, Args and
 magic16 / run4_of): checked exhaustively against integer division.
 
 The kernel replaces run-time divisions by per-launch values with
