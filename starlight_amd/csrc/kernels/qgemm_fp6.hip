@@ -238,6 +238,11 @@ __global__ __launch_bounds__(256) void split_fp6(const float* __restrict__ a, co
     const int er = mag_exp(block_max_u32(mx, scratch_u));
     if (threadIdx.x == 0) row_exp[r] = er;
     const uint64_t m = gridDim.x;
+    // The records a last block reads past the last superblock's (up to 127, in
+    // kPad) hold what was there before: without further digits, or they would
+    // choose how the rows beside them are summed.
+    if (r == m - 1 && threadIdx.x < 128)
+        *reinterpret_cast<uint2*>(records + (k / 128 * m + threadIdx.x) * kRecord + kScalesAt) = make_uint2(0u, 0u);
     // One plane of 16 elements' codes: half h of lane block b.
     const auto store = [](uint8_t* plane, uint32_t h, uint32_t b, const uint32_t (&c)[16]) {
         const uint32_t w0 = c[0] | c[1] << 6 | c[2] << 12 | c[3] << 18 | c[4] << 24 | c[5] << 30;
@@ -513,11 +518,13 @@ __global__ __launch_bounds__(kWave* WM* WN) __attribute__((amdgpu_waves_per_eu(M
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(hi[j][e] + lo[j][e], here[j], acc[i][j][e]);
         }
-        // Further digits: elements of a block 2^8 and more apart. The sum of a plane is still exact or close, the four low planes' together is not, and
+        // Further digits: elements of a block 2^8 and more apart. The sum of a
+        // plane is still exact or close, the four low planes' together is not, and
         // is cut always downwards (a bias of 5e-7 over 129 superblocks), so each
         // plane starts from zero here and f32 additions, which round to nearest,
-        // join them from the lowest on. (A row past m may show another row's
-        // flag: it reads row m - 1's further digits and stores nothing.)
+        // join them from the lowest on. (A row past m may show a row's flag of
+        // the next superblock: it reads row m - 1's further digits and stores
+        // nothing.)
         if (wide) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) {

@@ -202,6 +202,20 @@ def test_infinities_and_nan_stay_in_their_row(hip):
     assert_products(got[keep], a[keep], w[2])
 
 
+# The rows of a tile past the last one, whose records are not written, hold what an
+# earlier call left there: with and without further digits
+@pytest.mark.parametrize("m,n,k", [(17, 300, 512), (33, 140, 128), (65, 520, 1024)])
+def test_results_do_not_depend_on_earlier_calls(hip, m, n, k):
+    r = np.random.default_rng(m)
+    a = r.standard_normal((m, k)).astype(np.float32)
+    w = weight(hip, n, k, 128, r)
+    smooth = r.standard_normal((4 * m, k)).astype(np.float32)
+    run(hip, smooth, w)
+    first = run(hip, a, w)
+    run(hip, outliers(r, 4 * m, k, 1e4, "each 32")[0], w)
+    assert np.array_equal(first, run(hip, a, w))
+
+
 # A device that made no 6-bit copies: the fp16 route, which keeps 22 bits of an
 # element down to 2^-40 of its row's largest, whose superblock is 8 products summed
 # in f32, and which sums in slices for one weight and for several
